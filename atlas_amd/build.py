@@ -24,7 +24,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libatlas_kernels.so")
 
-SOURCES = ["gemv.hip", "skinny.hip", "attention.hip", "fused.hip", "errors.cpp", "runtime.cpp",
+SOURCES = ["gemv.hip", "skinny.hip", "prompt_gemm.hip", "attention.hip", "fused.hip", "errors.cpp", "runtime.cpp",
            "capi.cpp", "engine.cpp", "st_format.cpp", "loader.cpp", "blas.cpp"]
 
 

@@ -53,15 +53,11 @@ constexpr int kBatchLongAttnFrom = 512;
 constexpr int kPrefillChunk = 16;
 constexpr int kMaxRows = kPrefillChunk;
 // Prompt chunks of models whose GEMM inner dims are multiples of 128 go
-// through the tiled MFMA GEMM (gemm_rows_launch), up to this many rows
-// per step, replayed eagerly (the captured steps stop at kMaxRows rows).
+// through the tiled MFMA GEMM (gemm_rows_launch), replayed eagerly (the
+// captured steps stop at kMaxRows rows): up to kPrefillLib rows per step, of
+// which the fused attention's buffers hold kPrefillBig.  Above 128 rows the
+// chunk's attention runs on the matrix cores.
 constexpr int kPrefillBig = 128;
-// ... and up to this many rows per step in all: the library GEMM (bf16, int8)
-// takes them at once (at the 7B shapes the GEMMs of a layer cost 1.28 us per
-// prompt token at 127 rows, 0.87 at 255 and 0.68 at 511, bf16; a 2047-token
-// prompt took 76.8 ms in 512-row chunks and 68.9 in 1024), the tiled kernel
-// (int4) in 128-row launches; the chunk's attention then runs on the matrix
-// cores (above 128 rows).
 constexpr int kPrefillLib = 1024;
 
 struct DevMat {
@@ -1543,8 +1539,9 @@ ATLAS_API atlas_model* atlas_model_create(const atlas_model_config* cfg) {
         size_t need = 0;
         for (const auto& sh : shapes) {
             if (sh[1] % 32 == 0) need = std::max(need, skinny_partial_bytes(sh[0], nb, sh[1]));
-            if (m->big_prefill)
-                need = std::max(need, gemm_rows_partial_bytes(sh[0], kPrefillBig, sh[1]));
+            if (sh[1] % 128 == 0)                        // (prompt chunks stop before the lm_head)
+                need = std::max(need, gemm_rows_partial_bytes(
+                                          fmt, sh[0], m->big_prefill && &sh != &shapes[4] ? R : nb, sh[1]));
         }
         if (need && dalloc(m, (void**)&m->gemm_part, need)) return fail(m);
         m->gemm_part_bytes = need;

@@ -44,7 +44,7 @@ struct GemvArgs {
     size_t partial_bytes;    // ... their size
     // skinny_launch, host side: non-null with EPI_STORE and the caller's
     // partial buffer, a split-K launch of the 2-8-row direct-load kernels or
-    // of the tiled prompt GEMM (17-128 rows, one launch) leaves its partials
+    // of the prompt GEMMs (9+ rows) leaves its partials
     // in `partial` ([splits][N][M], summed in split order by the consumer)
     // and stores the split count here instead of launching the reduce; 0
     // when y was written.
@@ -68,11 +68,19 @@ int gemv_multi_launch(const GemvArgs& a, hipStream_t st);
 size_t skinny_partial_bytes(int M, int N, int K);    // split-K partials of (M, N, K)
 // y = the fixed-order sum of `splits` partials ([splits][N][M]), with a's epilogue
 int skinny_reduce_launch(const GemvArgs& a, const float* partial, int splits, hipStream_t st);
-// 17+ rows: the tiled MFMA GEMM (skinny_launch routes there; 128 rows per
-// launch) or, with a library context, the hipBLASLt prompt GEMM
+// whether the caller takes the split-K sum over (GemvArgs.defer_splits), and
+// where the partials go: its buffer or the calling thread's scratch
+bool skinny_defer_ok(const GemvArgs& a);
+int skinny_partial_for(const GemvArgs& a, size_t bytes, float** out);
+// Nine or more rows (2-8 of small matrices) of K % 128 == 0: the MFMA GEMMs of
+// prompt_gemm.hip (skinny_launch routes there) or, from 17 with a library context, the hipBLASLt prompt GEMM.
+// gemm_rows_ok: formats, alignment and strides they take; gemm_rows_fit: sizes
+// within their 32-bit offsets.  A call with needs_scratch false makes do
+// without a K split where the partials cannot be had.
 bool gemm_rows_ok(const GemvArgs& a);
-int gemm_rows_launch(const GemvArgs& a, hipStream_t st);
-size_t gemm_rows_partial_bytes(int M, int N, int K);
+bool gemm_rows_fit(const GemvArgs& a);
+int gemm_rows_launch(const GemvArgs& a, bool needs_scratch, hipStream_t st);
+size_t gemm_rows_partial_bytes(int fmt, int M, int N, int K);    // covers every smaller N
 // The bf16 and int8 prompt GEMMs through hipBLASLt (blas.cpp): X's rows split
 // into bf16 hi and lo rows (bf16 weights) or three int8 digit rows (int8
 // weights), one library GEMM of the weights against all of them (the weights

@@ -39,10 +39,9 @@
 
 #include "common.hpp"
 #include "gemv.hpp"
+#include "mfma.hpp"
 
 namespace atlas {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int SK_WAVES = 16;        // waves per block
 constexpr int SK_KTW = 8;           // max 32-k tiles per wave
@@ -64,11 +63,6 @@ __device__ __forceinline__ uint32_t split_part(float v, bool lo) {
 
 __device__ __forceinline__ uint32_t pack2(uint32_t lo16, uint32_t hi16) {
     return (lo16 & 0xFFFFu) | (hi16 << 16);
-}
-
-// two f32 with <= 8 significant bits -> packed bf16 pair (a low), exact
-__device__ __forceinline__ uint32_t pack_f32_pair(float a, float b) {
-    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
 
 // one lane's weights of one 32-k tile
@@ -515,19 +509,6 @@ __device__ __forceinline__ void rows_transpose4(uint32_t& r0, uint32_t& r1, uint
     r1 = q01[1];
     r2 = q23[0];
     r3 = q23[1];
-}
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// packed bf16 of (a, b): hi = truncation, lo = the rounded remainder
-__device__ __forceinline__ uint32_t bf16_hi2(float a, float b) {
-    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-}
-__device__ __forceinline__ uint32_t bf16_lo2(float a, float b) {
-    const float ra = a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
-    const float rb = b - __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
-    const bf16x2 v = {(__bf16)ra, (__bf16)rb};
-    return __builtin_bit_cast(uint32_t, v);
 }
 
 constexpr int SKD_KTW = 8;          // 32-k tiles per wave
@@ -1021,23 +1002,39 @@ __global__ __launch_bounds__(1024) void skinny_lds_kernel(GemvArgs a) {
     }
 }
 
+// (eight partials of an element are in flight at once; they are added in split order)
 __global__ __launch_bounds__(256) void skinny_reduce_kernel(GemvArgs a, const float* __restrict__ partial,
                                                             int splitk) {
     const int M = a.M, N = a.N;
     const int m_out = a.epi == EPI_SILU_MUL ? M / 2 : M;
-    const long total = (long)N * m_out;
+    const long total = (long)N * m_out, plane = (long)N * M;
     for (long i = blockIdx.x * 256L + threadIdx.x; i < total; i += (long)gridDim.x * 256) {
         const int n = (int)(i / m_out), mo = (int)(i % m_out);
         if (a.epi == EPI_SILU_MUL) {
-            float gsum = 0.f, usum = 0.f;
-            for (int s = 0; s < splitk; ++s) {
-                gsum += partial[((long)s * N + n) * M + 2 * mo];
-                usum += partial[((long)s * N + n) * M + 2 * mo + 1];
+            typedef float f32x2 __attribute__((ext_vector_type(2)));
+            const float* p = partial + (long)n * M + 2 * mo;
+            f32x2 sum = {0.f, 0.f};
+            for (int s0 = 0; s0 < splitk; s0 += 8) {
+                f32x2 v[8];
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    v[s] = *reinterpret_cast<const f32x2*>(p + min(s0 + s, splitk - 1) * plane);
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    if (s0 + s < splitk) sum += v[s];
             }
-            a.y[n * a.y_stride_n + (long)mo * a.y_stride_m] = gsum / (1.0f + expf(-gsum)) * usum;
+            a.y[n * a.y_stride_n + (long)mo * a.y_stride_m] = sum.x / (1.0f + expf(-sum.x)) * sum.y;
         } else {
+            const float* p = partial + (long)n * M + mo;
             float sum = 0.f;
-            for (int s = 0; s < splitk; ++s) sum += partial[((long)s * N + n) * M + mo];
+            for (int s0 = 0; s0 < splitk; s0 += 8) {
+                float v[8];
+#pragma unroll
+                for (int s = 0; s < 8; ++s) v[s] = p[min(s0 + s, splitk - 1) * plane];
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    if (s0 + s < splitk) sum += v[s];
+            }
             a.y[n * a.y_stride_n + (long)mo * a.y_stride_m] = sum;
         }
     }
@@ -1055,14 +1052,14 @@ int skinny_reduce_launch(const GemvArgs& a, const float* partial, int splits, hi
 
 // The caller takes the split-K sum over (GemvArgs.defer_splits): plain
 // stores into its own partial buffer only.
-static bool defer_ok(const GemvArgs& a) {
+bool skinny_defer_ok(const GemvArgs& a) {
     return a.defer_splits && a.epi == EPI_STORE && a.partial && a.y_stride_m == 1 &&
            a.y_stride_n == a.M;
 }
 
 // Split-K partials: the caller's buffer (GemvArgs.partial, e.g. a model's,
 // which a captured step may point at) or the calling thread's scratch.
-static int partial_for(const GemvArgs& a, size_t bytes, float** out) {
+int skinny_partial_for(const GemvArgs& a, size_t bytes, float** out) {
     if (a.partial) {
         ATLAS_REQUIRE(bytes <= a.partial_bytes, "split-K partials: %zu bytes needed, %zu given",
                       bytes, a.partial_bytes);
@@ -1114,7 +1111,7 @@ static int launch_skinny(const GemvArgs& a, hipStream_t st) {
     if (bx > n_tiles) bx = n_tiles;
     float* partial = nullptr;
     if (splits > 1) {
-        int rc = partial_for(a, (size_t)splits * a.N * a.M * sizeof(float), &partial);
+        int rc = skinny_partial_for(a, (size_t)splits * a.N * a.M * sizeof(float), &partial);
         if (rc) return rc;
     }
     int cpb_shift = 0;
@@ -1205,7 +1202,7 @@ static int launch_skinny_i4d(const GemvArgs& a, hipStream_t st) {
     const bool sv = a.cpb == 1 && a.bpr % 4 == 0 && kt_total % 4 == 0 && ((uintptr_t)a.scales & 15) == 0;
     float* partial = nullptr;
     if (splits > 1) {
-        const int rc = partial_for(a, (size_t)splits * a.N * a.M * sizeof(float), &partial);
+        const int rc = skinny_partial_for(a, (size_t)splits * a.N * a.M * sizeof(float), &partial);
         if (rc) return rc;
     }
     int cpb_shift = 0;
@@ -1220,7 +1217,7 @@ static int launch_skinny_i4d(const GemvArgs& a, hipStream_t st) {
     default: i4d_go<8, 4>(a, sv, grid, st, partial, kt_split, cpb_shift); break;
     }
     ATLAS_LAUNCH_CHECK("skinny int4");
-    if (splits > 1 && defer_ok(a)) {
+    if (splits > 1 && skinny_defer_ok(a)) {
         *a.defer_splits = splits;
         return ATLAS_OK;
     }
@@ -1253,7 +1250,7 @@ static int launch_skinny_d(const GemvArgs& a, hipStream_t st) {
     const I4dPlan pl = i4d_plan(a.M, a.K, device_cu_count());
     float* partial = nullptr;
     if (pl.splits > 1) {
-        const int rc = partial_for(a, (size_t)pl.splits * a.N * a.M * sizeof(float), &partial);
+        const int rc = skinny_partial_for(a, (size_t)pl.splits * a.N * a.M * sizeof(float), &partial);
         if (rc) return rc;
     }
     const dim3 grid(pl.bx, pl.splits);
@@ -1266,7 +1263,7 @@ static int launch_skinny_d(const GemvArgs& a, hipStream_t st) {
     default: d_go<FMT, 8, 8>(a, grid, st, partial, pl.kt_split); break;
     }
     ATLAS_LAUNCH_CHECK(FMT == WF_BF16 ? "skinny bf16" : "skinny int8");
-    if (pl.splits > 1 && defer_ok(a)) {
+    if (pl.splits > 1 && skinny_defer_ok(a)) {
         *a.defer_splits = pl.splits;
         return ATLAS_OK;
     }
@@ -1298,28 +1295,7 @@ static int launch_skinny_lds(const GemvArgs& a, hipStream_t st) {
     return ATLAS_OK;
 }
 
-// ---------------------------------------------------------------------------
-// Prompt chunks: Y[n, m] = sum_k W[m, k] X[n, k] for 17 <= N <= 128 rows of
-// bf16, int8 or int4 weights (dequantised to exact bf16 operands as in
-// skinny_kernel: int8 row scales in the epilogue, int4 block scales on each
-// 32-k step's product).  Same operand roles and hi/lo split as skinny_kernel, but
-// every A fragment now feeds many weight tiles, so the matrix cores do the
-// work and the weights stream once per chunk:
-//  * a 256-thread block owns 128 weight rows (wave w: rows 32 w .. +31, two
-//    B fragments per 32-k step) and all NT 16-row tiles of X;
-//  * A fragments (X hi and lo, bf16) go through LDS, 2 k steps per chunk,
-//    double-buffered: each chunk's global reads are issued one chunk ahead
-//    and converted after the MFMAs of the current one;
-//  * B fragments (16 B per lane, straight from HBM) are refilled in place
-//    four k steps ahead, as soon as each has become an operand;
-//  * K splits over blockIdx.y when the row blocks alone leave CUs idle;
-//    partials are summed by skinny_reduce_kernel in a fixed order.
-// Per 32-k step a wave issues NT x 2 x 2 MFMAs (tiles x B fragments x hi/lo).
-constexpr int GR_ROWS = 128;        // weight rows per block
-constexpr int GR_MAX_N = 128;       // activation rows per launch
-// (k step, tile) items whose A fragments are read ahead of the current one
-constexpr int GR_AHEAD = 4;
-
+// ---- the element-wise halves of the hipBLASLt prompt GEMM ---------------------
 // hi / lo bf16 parts of 8 floats, packed as MFMA operands: hi = the high
 // halves (truncation), lo = the remainder rounded to nearest even (one
 // hardware conversion per pair)
@@ -1328,292 +1304,6 @@ __device__ __forceinline__ void split8(const f32x4 p0, const f32x4 p1, u32x4& hi
     lo = u32x4{bf16_lo2(p0.x, p0.y), bf16_lo2(p0.z, p0.w), bf16_lo2(p1.x, p1.y), bf16_lo2(p1.z, p1.w)};
 }
 
-// int4 at eight tiles runs one block per CU: its per-step scaled products
-// need ~370 registers (spilled 27 at two blocks per CU), and one 128-row
-// launch that streams the weights once beats two 64-row launches that
-// stream them twice (127-token int4 prefill 14.1 -> 12.6 ms)
-template <int FMT, int NT>
-__global__ __launch_bounds__(256, (FMT == WF_I4 && NT == 8) ? 1 : 2) void gemm_rows_kernel(GemvArgs a, float* __restrict__ partial,
-                                                           int steps_per_split, int cpb_shift) {
-    constexpr int ITEMS = 2 * NT * 64 / 256;      // A items (8 floats) per thread per chunk
-    __shared__ u32x4 As[2][2][NT][2][64];         // [buf][k step][tile][hi/lo][lane]
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = lane >> 4, li = lane & 15;
-    const int M = a.M, N = a.N;
-    const int s0 = blockIdx.y * steps_per_split;
-    const int s1 = min(a.K / 32, s0 + steps_per_split);   // s1 - s0: a multiple of 4
-    const int m0 = blockIdx.x * GR_ROWS + wave * 32;
-    SkRow wrow[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) wrow[j] = sk_row<FMT>(a, min(m0 + 16 * j + li, M - 1));
-    // A item q of this thread: (k step st, tile t, row i, k group gg) of a chunk
-    auto xload = [&](int chunk, int q, f32x4& p0, f32x4& p1) {
-        const int it = (int)threadIdx.x + 256 * q;
-        const int gg = it & 3, ii = (it >> 2) & 15, t = (it >> 6) % NT, st = it / (64 * NT);
-        const int n = t * 16 + ii;
-        const long k = (long)(s0 + 2 * chunk + st) * 32 + 8 * gg;
-        const float* xr = a.x + (long)min(n, N - 1) * a.x_stride_n + k;
-        p0 = *reinterpret_cast<const f32x4*>(xr);
-        p1 = *reinterpret_cast<const f32x4*>(xr + 4);
-        if (n >= N) p0 = p1 = f32x4{0.f, 0.f, 0.f, 0.f};
-    };
-    auto xstore = [&](int buf, int q, const f32x4& p0, const f32x4& p1) {
-        const int it = (int)threadIdx.x + 256 * q;
-        const int gg = it & 3, ii = (it >> 2) & 15, t = (it >> 6) % NT, st = it / (64 * NT);
-        u32x4 hi, lo;
-        split8(p0, p1, hi, lo);
-        As[buf][st][t][0][16 * gg + ii] = hi;
-        As[buf][st][t][1][16 * gg + ii] = lo;
-    };
-
-    const int nsteps = s1 - s0;                   // k steps of this split
-    const int nchunks = nsteps / 2;
-    f32x4 xr0[ITEMS], xr1[ITEMS];                 // the next chunk's A items
-#pragma unroll
-    for (int q = 0; q < ITEMS; ++q) xload(0, q, xr0[q], xr1[q]);
-#pragma unroll
-    for (int q = 0; q < ITEMS; ++q) xstore(0, q, xr0[q], xr1[q]);
-#pragma unroll
-    for (int q = 0; q < ITEMS; ++q) xload(min(1, nchunks - 1), q, xr0[q], xr1[q]);
-    SkFrag<FMT> B[4][2];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) sk_load<FMT>(wrow[j], s0 + u, g, cpb_shift, B[u][j]);
-    __syncthreads();
-
-    f32x4 acc[NT][2];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // One chunk (k steps 2c, 2c+1; B slots u0, u0+1) as 2 NT items (k step,
-    // tile) in order.  Each item's A fragments are read from LDS GR_AHEAD
-    // items before its MFMAs, and X item q of chunk c+1 is split into the
-    // other LDS buffer (then its registers take chunk c+2's item) between the
-    // MFMAs of items 4q and 4q+1; scheduling barriers hold that order, so the
-    // LDS latency and the split's VALU work overlap the matrix cores instead
-    // of preceding them.
-    auto chunk_body = [&](int c, int buf, int u0) {
-        const int cn = min(c + 2, nchunks - 1);
-        if constexpr (FMT == WF_I4 && NT == 8) {
-            // int4 at eight tiles keeps its per-step products in registers
-            // already (one block per CU); the items' extra live fragments
-            // would spill, so its A fragments are read as used, and X item q
-            // of the next chunk is split between k step 0's tiles 2q and 2q+1
-#pragma unroll
-            for (int st = 0; st < 2; ++st) {
-                const int u = u0 + st, s = s0 + 2 * c + st;
-                bf16x8 bb[2];
-                float ss[2];
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    bb[j] = sk_operand<FMT>(B[u][j]);
-                    ss[j] = B[u][j].s;
-                    sk_load<FMT>(wrow[j], min(s + 4, s1 - 1), g, cpb_shift, B[u][j]);   // refill: step s + 4
-                }
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    if (st == 0 && (t & 1)) {
-                        const int q = t >> 1;
-                        if (c + 1 < nchunks) xstore(buf ^ 1, q, xr0[q], xr1[q]);
-                        xload(cn, q, xr0[q], xr1[q]);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                    const bf16x8 xh = __builtin_bit_cast(bf16x8, As[buf][st][t][0][lane]);
-                    const bf16x8 xl = __builtin_bit_cast(bf16x8, As[buf][st][t][1][lane]);
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, bb[j], f32x4{0.f, 0.f, 0.f, 0.f},
-                                                                          0, 0, 0);
-                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, bb[j], d, 0, 0, 0);
-                        acc[t][j] += d * ss[j];
-                    }
-                }
-            }
-            __syncthreads();
-            return;
-        }
-        constexpr int NI = 2 * NT, D = GR_AHEAD < NI ? GR_AHEAD : NI;
-        bf16x8 ah[NI], al[NI];
-        bf16x8 b[2][2];
-        float sc[2][2];
-        auto aread = [&](int i) {
-            const int st = i / NT, t = i % NT;
-            ah[i] = __builtin_bit_cast(bf16x8, As[buf][st][t][0][lane]);
-            al[i] = __builtin_bit_cast(bf16x8, As[buf][st][t][1][lane]);
-        };
-        auto bprep = [&](int st) {
-            const int u = u0 + st, s = s0 + 2 * c + st;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                b[st][j] = sk_operand<FMT>(B[u][j]);
-                if constexpr (FMT == WF_BF16) asm volatile("" : "+v"(b[st][j]));
-                sc[st][j] = 1.0f;
-                if constexpr (FMT == WF_I4) sc[st][j] = B[u][j].s;
-                sk_load<FMT>(wrow[j], min(s + 4, s1 - 1), g, cpb_shift, B[u][j]);   // refill: step s + 4
-            }
-        };
-        bprep(0);
-#pragma unroll
-        for (int i = 0; i < D; ++i) aread(i);
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            if (i + D < NI) aread(i + D);
-            if (i == NT) bprep(1);
-            if (i % 4 == 1) {
-                const int q = i / 4;                  // ITEMS = NI / 4
-                if (c + 1 < nchunks) xstore(buf ^ 1, q, xr0[q], xr1[q]);
-                xload(cn, q, xr0[q], xr1[q]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            const int st = i / NT, t = i % NT;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if constexpr (FMT == WF_I4) {
-                    // the step is one scale block of the lane's row
-                    f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], b[st][j],
-                                                                      f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], b[st][j], d, 0, 0, 0);
-                    acc[t][j] += d * sc[st][j];
-                } else {
-                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], b[st][j], acc[t][j], 0, 0, 0);
-                    acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], b[st][j], acc[t][j], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
-    };
-    // block-uniform trip count: four k steps (two chunks, buffers 0 and 1)
-    for (int c = 0; c < nchunks; c += 2) {
-        chunk_body(c, 0, 0);
-        chunk_body(c + 1, 1, 2);
-    }
-
-    // ---- epilogue: lane (g, li) holds D[4 g + v][li] of tile (t, j)
-    const bool split_out = gridDim.y > 1;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int m = m0 + 16 * j + li;
-            float rs = 1.0f;                                   // int8 row scale
-            if constexpr (FMT == WF_I8) rs = a.scales[min(m, M - 1)];
-            const float vals[4] = {acc[t][j].x * rs, acc[t][j].y * rs, acc[t][j].z * rs,
-                                   acc[t][j].w * rs};
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int n = t * 16 + 4 * g + v;
-                const float val = vals[v];
-                if (split_out) {
-                    if (n < N && m < M) partial[((long)blockIdx.y * N + n) * M + m] = val;
-                } else if (a.epi == EPI_SILU_MUL) {
-                    const float up = __shfl_xor(val, 1, 64);   // rows (2i, 2i+1) = (gate, up)
-                    if ((m & 1) == 0 && n < N && m + 1 < M)
-                        a.y[n * a.y_stride_n + (long)(m >> 1) * a.y_stride_m] =
-                            val / (1.0f + expf(-val)) * up;
-                } else if (n < N && m < M) {
-                    a.y[n * a.y_stride_n + (long)m * a.y_stride_m] = val;
-                }
-            }
-        }
-}
-
-// K splits of a rows launch: enough (row block, split) blocks for one per
-// CU, each split a multiple of four k steps.  (Two per CU, the occupancy
-// limit, measured 3% slower over the 7B GEMMs at 128 rows and 8% at 64:
-// the extra partials and reduce cost more than the second block gains.)
-// int4 (one block per CU at eight tiles) takes no K split once its row blocks
-// alone cover 60% of the CUs: a second split's blocks would run as a second
-// round, and its partials and reduce cost ~7 us (7B gate/up, 127-token int4
-// prefill 12.0 -> 11.8 ms).  For bf16 and int8 (two blocks per CU) the split
-// stays faster (8.0 against 7.8 ms, 8.1 against 7.5 ms).
-static void gemm_rows_split(int M, int K, int& splits, int& steps, int fmt = WF_BF16) {
-    const int bx = (M + GR_ROWS - 1) / GR_ROWS, ksteps = K / 32;
-    const int cus = device_cu_count();
-    int want = fmt == WF_I4 && 5 * bx >= 3 * cus ? 1 : (cus + bx - 1) / bx;
-    want = std::max(1, std::min(want, ksteps / 4));
-    steps = ((ksteps + want - 1) / want + 3) / 4 * 4;
-    splits = (ksteps + steps - 1) / steps;
-}
-
-// a: after gemv_fill_int4_index (int4 bpr / cpb)
-bool gemm_rows_ok(const GemvArgs& a) {
-    const uintptr_t wa = (uintptr_t)a.w;
-    const bool fmt_ok =
-        a.fmt == WF_BF16 ? (wa & 15) == 0 && (a.ldw == 0 || a.ldw % 16 == 0)
-        : a.fmt == WF_I8 ? a.scales && (wa & 7) == 0 && (a.ldw == 0 || a.ldw % 8 == 0)
-        : a.fmt == WF_I4 ? a.scales && (wa & 3) == 0 && a.ldw == 0 && a.block % 32 == 0 &&
-                               a.bpr > 0 && (a.cpb & (a.cpb - 1)) == 0
-                         : false;
-    return fmt_ok && a.N > 16 && a.K % 128 == 0 && a.M > 0 &&
-           a.x_stride_k == 1 && a.x_stride_n % 4 == 0 && ((uintptr_t)a.x & 15) == 0 &&
-           (a.epi == EPI_STORE || (a.epi == EPI_SILU_MUL && a.M % 2 == 0));
-}
-
-// 2, 4 or 8 16-row tiles per launch; more are refused rather than left
-// unwritten (gemm_rows_launch splits chunks above 128 rows)
-template <int FMT>
-static int gemm_rows_go(const GemvArgs& a, float* partial, dim3 grid, int steps, int cpb_shift,
-                        hipStream_t st) {
-    const int nt = (a.N + 15) / 16;
-    if (nt <= 2)
-        hipLaunchKernelGGL((gemm_rows_kernel<FMT, 2>), grid, dim3(256), 0, st, a, partial, steps, cpb_shift);
-    else if (nt <= 4)
-        hipLaunchKernelGGL((gemm_rows_kernel<FMT, 4>), grid, dim3(256), 0, st, a, partial, steps, cpb_shift);
-    else if (nt <= 8)
-        hipLaunchKernelGGL((gemm_rows_kernel<FMT, 8>), grid, dim3(256), 0, st, a, partial, steps, cpb_shift);
-    else {
-        set_error(ATLAS_EUNSUPPORTED, "gemm rows: a launch takes at most 128 rows (got %d)", a.N);
-        return ATLAS_EUNSUPPORTED;
-    }
-    return ATLAS_OK;
-}
-
-size_t gemm_rows_partial_bytes(int M, int N, int K) {
-    int splits, steps;
-    gemm_rows_split(M, K, splits, steps);
-    if (splits <= 1) return 0;
-    return (size_t)splits * N * M * sizeof(float);
-}
-
-// one launch (+ split-K reduce, unless a.defer_splits takes the split count)
-// over all a.N <= 128 rows
-static int gemm_rows_part(const GemvArgs& a, hipStream_t st) {
-    int splits, steps;
-    gemm_rows_split(a.M, a.K, splits, steps, a.fmt);
-    float* partial = nullptr;
-    if (splits > 1) {
-        int rc = partial_for(a, (size_t)splits * a.N * a.M * sizeof(float), &partial);
-        if (rc) return rc;
-    }
-    const dim3 grid((a.M + GR_ROWS - 1) / GR_ROWS, splits);
-    int cpb_shift = 0;
-    while ((1 << cpb_shift) < a.cpb) ++cpb_shift;
-    int rc;
-    if (a.fmt == WF_BF16) rc = gemm_rows_go<WF_BF16>(a, partial, grid, steps, cpb_shift, st);
-    else if (a.fmt == WF_I8) rc = gemm_rows_go<WF_I8>(a, partial, grid, steps, cpb_shift, st);
-    else rc = gemm_rows_go<WF_I4>(a, partial, grid, steps, cpb_shift, st);
-    if (rc) return rc;
-    ATLAS_LAUNCH_CHECK("gemm_rows");
-    if (splits > 1 && defer_ok(a)) {
-        *a.defer_splits = splits;             // the consumer sums the partials
-        return ATLAS_OK;
-    }
-    if (splits > 1) {
-        const long m_out = a.epi == EPI_SILU_MUL ? a.M / 2 : a.M;
-        long rb = ((long)a.N * m_out + 255) / 256;
-        if (rb > 4096) rb = 4096;
-        hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)rb), dim3(256), 0, st, a, partial,
-                           splits);
-        ATLAS_LAUNCH_CHECK("gemm_rows_reduce");
-    }
-    return ATLAS_OK;
-}
-
-// ---- the element-wise halves of the hipBLASLt prompt GEMM ---------------------
 // Thread per 8 consecutive k of one row: the split of the tiled kernel
 // (hi = the top 16 bits, lo = the rest rounded to nearest even).
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, long sn, int N,
@@ -1809,22 +1499,6 @@ int combine_rows_launch(const float* d, int N, int M, int epi, float* y, long ys
     return ATLAS_OK;
 }
 
-int gemm_rows_launch(const GemvArgs& a, hipStream_t st) {
-    ATLAS_REQUIRE(gemm_rows_ok(a), "gemm rows: unsupported shape (fmt %d, n %d, k %d)", a.fmt, a.N,
-                  a.K);
-    const int cap = GR_MAX_N;
-    for (int n0 = 0; n0 < a.N; n0 += cap) {
-        GemvArgs p = a;
-        p.N = std::min(cap, a.N - n0);
-        p.x = a.x + (long)n0 * a.x_stride_n;
-        p.y = a.y + (long)n0 * a.y_stride_n;
-        if (a.N > cap) p.defer_splits = nullptr;   // the parts share one partial buffer
-        int rc = gemm_rows_part(p, st);
-        if (rc) return rc;
-    }
-    return ATLAS_OK;
-}
-
 template <int FMT>
 static int launch_skinny_n(const GemvArgs& a, hipStream_t st) {
     return a.N > 8 ? launch_skinny<FMT, 2>(a, st) : launch_skinny<FMT, 1>(a, st);
@@ -1843,10 +1517,58 @@ static bool halves_pay(const GemvArgs& a) {
     return a.fmt == WF_BF16 && a.K > 4096;
 }
 
+// Whether this shape's rows have always needed split-K scratch, so that a call
+// that cannot have it is refused rather than run without a split.
+static bool rows_need_scratch(const GemvArgs& a) {
+    const int cus = device_cu_count();
+    if (a.N > 16) {
+        const int bx = (a.M + 127) / 128;
+        return bx < cus && !(a.fmt == WF_I4 && 5 * bx >= 3 * cus) && a.K >= 256;
+    }
+    if (a.N > 8 && !halves_pay(a)) return skinny_splits(a.K, a.N) > 1;
+    if (a.fmt != WF_I4 && a.K <= 4096) return false;
+    return i4d_plan(a.M, a.K, cus).splits > 1;
+}
+
+// Which rows take the few-rows and tiled GEMMs of prompt_gemm.hip (where
+// gemm_rows_ok): all from nine up; at the 7B shapes and 13 rows they take
+// 0.55-0.9x the time of the kernels below (bf16 W_down 41.5 -> 22.5 us, gate/up
+// 47.9 -> 38.6, int8 29.4 -> 16.3 and 39.9 -> 24.1, int4 25.3 -> 15.6 and
+// 29.3 -> 26.5).  Of 2-8 rows those of small matrices, where the kernels below
+// leave CUs idle (4 rows, us: bf16 2048 x 8192 14.6 -> 10.2, 8192 x 2048
+// 11.3 -> 9.3, 640 x 640 7.5 -> 4.1; int8 9.2 -> 9.1, 9.5 -> 8.7, 6.6 -> 4.5);
+// from there up their streaming is the faster one (bf16 12288 x 4096 19.7
+// against 21.6, int8 13.4 against 15.6), and int4's at nearly every size
+// (2048 x 8192 9.0 against 9.7, 3072 x 768 + 768 x 1536 15.4 against 16.1).
+// Two bf16 rows of K <= 4096 keep the multi-row GEMV, whose products are f32.
+static bool few_rows_pay(const GemvArgs& a) {
+    if (a.N >= 9) return true;
+    const long el = (long)a.M * a.K;
+    if (a.fmt == WF_I8) return a.N >= 2 && el <= 1L << 24;
+    return a.fmt == WF_BF16 && el <= 1L << 24 && (a.N >= 3 || (a.N == 2 && a.K > 4096));
+}
+
 int skinny_launch(const GemvArgs& a_in, hipStream_t st) {
     GemvArgs a = a_in;
     if (a.defer_splits) *a.defer_splits = 0;
     gemv_fill_int4_index(a);
+    const bool rows_ok = few_rows_pay(a) && a.w && a.x && a.y && gemm_rows_ok(a);
+    if (rows_ok && a.N > 16 && a.blas && (a.fmt == WF_BF16 || (a.fmt == WF_I8 && a.K <= kDigitsMaxK)))
+        return blas_rows_launch(a.blas, a, st);
+    if (rows_ok && gemm_rows_fit(a) && (a.N > 16 || gemv_pitch_ok(a)))
+        return gemm_rows_launch(a, rows_need_scratch(a), st);
+    if (rows_ok && a.N > 16) {               // rows too long for their offsets: 16 at a time
+        for (int n0 = 0; n0 < a.N; n0 += 16) {
+            GemvArgs p = a;
+            p.defer_splits = nullptr;
+            p.N = std::min(16, a.N - n0);
+            p.x = a.x + (long)n0 * a.x_stride_n;
+            p.y = a.y + (long)n0 * a.y_stride_n;
+            const int rc = skinny_launch(p, st);
+            if (rc) return rc;
+        }
+        return ATLAS_OK;
+    }
     if (halves_pay(a)) {
         const int n0 = (a.N + 1) / 2;
         GemvArgs h = a;
@@ -1860,10 +1582,6 @@ int skinny_launch(const GemvArgs& a_in, hipStream_t st) {
         return skinny_launch(h, st);
     }
     a.x_vec = a.x_stride_k == 1 && a.x_stride_n % 4 == 0 && ((uintptr_t)a.x & 15) == 0;
-    if (a.N > 16 && gemm_rows_ok(a))
-        return a.blas && (a.fmt == WF_BF16 || (a.fmt == WF_I8 && a.K <= kDigitsMaxK))
-                   ? blas_rows_launch(a.blas, a, st)
-                   : gemm_rows_launch(a, st);
     ATLAS_REQUIRE(a.N >= 1 && a.N <= 16, "skinny: N=%d outside 1..16 (17+ rows need K %% 128 == 0 "
                   "and, for int4, blocks of 32 * 2^j)", a.N);
     ATLAS_REQUIRE(a.w && a.x && a.y, "skinny: null pointer");
