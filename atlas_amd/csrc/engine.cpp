@@ -237,10 +237,13 @@ int gemv(atlas_model* m, const DevMat& w, const float* x, float* y, int epi) {
     return gemv_launch(gemv_args(w, x, y, epi), m->st);
 }
 
+// f32x: activations with all their 24 bits (bf16 / int8 weights; int4's own
+// batch-1 products hold fewer)
 int skinny(atlas_model* m, const DevMat& w, const float* x, float* y, int n, int epi,
-           int* defer_splits = nullptr) {
+           int* defer_splits = nullptr, bool f32x = false) {
     GemvArgs a = gemv_args(w, x, y, epi);
     a.defer_splits = defer_splits;
+    a.f32x = f32x && w.fmt != WF_I4;
     a.N = n;
     a.x_stride_n = w.cols;
     a.x_stride_k = 1;
@@ -392,10 +395,13 @@ int enqueue_attn_long(atlas_model* m, const LayerW& L) {
     return attn_launch(a, m->attn_splits_long, m->st);
 }
 
-// GU of the fused step: x'_l = x_l + rmsnorm(y1) * attn_norm_l materialised
-// into xb, then h = silu(gate) * up in the epilogue.
+// GU of the fused step: x'_l = x_l + rmsnorm(y1) * attn_norm_l (pre-norm: x_l + y1,
+// its norm by ffn_norm_l as the input) materialised into xb, then
+// h = silu(gate) * up in the epilogue.
 int enqueue_gu_fused(atlas_model* m, const LayerW& L) {
-    GemvArgs gu = pro_args(L.gu, m->x, m->h, PRO_RESNORM, m->y, L.attn_norm, m->cfg.rms_eps, m->xb);
+    const bool post = m->cfg.post_norm;
+    GemvArgs gu = pro_args(L.gu, m->x, m->h, post ? PRO_RESNORM : PRO_ADDNORM, m->y,
+                           post ? L.attn_norm : L.ffn_norm, m->cfg.rms_eps, m->xb);
     gu.epi = EPI_SILU_MUL;
     return gemv_launch(gu, m->st);
 }
@@ -405,18 +411,21 @@ int enqueue_down_fused(atlas_model* m, const LayerW& L) {
     return gemv(m, L.down, m->h, m->y2, EPI_STORE);
 }
 
-// The post-norm decode step with the norms folded into the GEMV prologues
-// and one attention launch per layer (5 launches per layer):
+// The decode step with the norms folded into the GEMV prologues and one
+// attention launch per layer (5 launches per layer):
 //   QKV    x_l = x'_{l-1} + rmsnorm(y2) * ffn_norm_{l-1}   (layer 0: embedding)
 //   ATTN   QK-norm + RoPE + KV write + split-K attention + merge
 //   WO     y1 = W_o att
 //   GU     x'_l = x_l + rmsnorm(y1) * attn_norm_l;  h = silu(gate) * up
 //   DOWN   y2 = W_down h
-// x_l lives in m->x, x'_l in m->xb.
+// x_l lives in m->x, x'_l in m->xb.  Pre-norm models (lib.rs:994-1005) add
+// plainly, x_l = x'_{l-1} + y2 and x'_l = x_l + y1, and QKV, GU and the lm_head
+// take the norm of the sum (attn_norm_l, ffn_norm_l, final_norm).
 int enqueue_step_fused(atlas_model* m, int mode, bool long_ctx) {
     const atlas_model_config& c = m->cfg;
     const int d = c.d_model;
     const float eps = c.rms_eps;
+    const bool post = c.post_norm;
     RopeRowArgs rr;
     rr.pos_dev = m->pos_dev; rr.cos_tab = m->cos_tab; rr.sin_tab = m->sin_tab; rr.half = m->hd / 2;
     rr.out = long_ctx ? nullptr : m->rope_row;
@@ -424,7 +433,11 @@ int enqueue_step_fused(atlas_model* m, int mode, bool long_ctx) {
     for (int li = 0; li < c.n_layers; ++li) {
         LayerW& L = m->L[li];
         if (li == 0)
-            TRY(gemv_launch(pro_args(L.qkv, m->x, m->qkv, PRO_X, nullptr, nullptr, 0.f, nullptr), m->st));
+            TRY(gemv_launch(pro_args(L.qkv, m->x, m->qkv, post ? PRO_X : PRO_RMSNORM, nullptr,
+                                     post ? nullptr : L.attn_norm, eps, nullptr), m->st));
+        else if (!post)
+            TRY(gemv_launch(pro_args(L.qkv, m->xb, m->qkv, PRO_ADDNORM, m->y2, L.attn_norm, eps, m->x),
+                            m->st));
         else
             TRY(gemv_launch(pro_args(L.qkv, m->xb, m->qkv, PRO_RESNORM, m->y2, m->L[li - 1].ffn_norm,
                                      eps, m->x), m->st));
@@ -464,7 +477,9 @@ int enqueue_step_fused(atlas_model* m, int mode, bool long_ctx) {
     GemvArgs h = pro_args(m->lm_head, m->xb, m->logits, PRO_RESNORM_NORM, m->y2,
                           m->L[c.n_layers - 1].ffn_norm, eps, hook_last);
     h.pro_w2 = m->final_norm;
-    if (!gemv_resnorm_norm_ok(h)) {
+    if (!post) {
+        h = pro_args(m->lm_head, m->xb, m->logits, PRO_ADDNORM, m->y2, m->final_norm, eps, hook_last);
+    } else if (!gemv_n2_ok(h)) {
         TRY(residual_rmsnorm_launch(m->xb, m->y2, m->L[c.n_layers - 1].ffn_norm, d, 1, d, eps,
                                     m->st));
         if (hook_last) TRY(ew_launch(EW_COPY, m->xb, nullptr, hook_last, 0.f, d, m->st));
@@ -1053,9 +1068,9 @@ int set_tensor_dev(atlas_model* m, int kind, int layer, const void* src, int src
 // ---- the ragged batch step ----------------------------------------------------
 // n rows of activations through w: the batch-1 GEMV for one row, the skinny
 // launcher for 2..16 (the multi-row GEMV for 2-3 rows, MFMA tiles above)
-int bmm(atlas_model* m, const DevMat& w, const float* x, float* y, int n, int epi) {
+int bmm(atlas_model* m, const DevMat& w, const float* x, float* y, int n, int epi, bool f32x = false) {
     if (n == 1) return gemv(m, w, x, y, epi);
-    return skinny(m, w, x, y, n, epi);
+    return skinny(m, w, x, y, n, epi, nullptr, f32x);
 }
 
 // y = w . x rows, then x += rmsnorm(y) * norm_w: where the GEMM splits K
@@ -1137,6 +1152,8 @@ int batch_step(atlas_model* m, int n, const std::vector<int>& slots, bool long_c
                bool prompt_chunk = false) {
     const atlas_model_config& c = m->cfg;
     const bool with_head = !prompt_chunk;
+    // a pre-norm model's prompt keeps the 24-bit activations of its decode step
+    const bool f32x = prompt_chunk && !c.post_norm;
     const int d = c.d_model;
     const int bfmt = prompt_chunk && long_ctx ? blas_chunk(m, n) : 0;
     const bool bc = bfmt != 0, b8 = bfmt == WF_I8;
@@ -1158,7 +1175,7 @@ int batch_step(atlas_model* m, int n, const std::vector<int>& slots, bool long_c
         // QKV GEMM's split-K partials in place of the reduce launch
         int qkv_splits = 0;
         if (bc) TRY(blas_gemm(m, L.qkv, n));
-        else if (m->fused && long_ctx && n > 1) TRY(skinny(m, L.qkv, xin, m->qkv, n, EPI_STORE, &qkv_splits));
+        else if (m->fused && long_ctx && n > 1) TRY(skinny(m, L.qkv, xin, m->qkv, n, EPI_STORE, &qkv_splits, f32x));
         else TRY(bmm(m, L.qkv, xin, m->qkv, n, EPI_STORE));
         QkvPostArgs q{};
         if (qkv_splits > 0) {
@@ -1279,11 +1296,11 @@ int batch_step(atlas_model* m, int n, const std::vector<int>& slots, bool long_c
             TRY(bmm(m, L.gu, m->x, m->h, n, EPI_SILU_MUL));
             TRY(bmm_resnorm(m, L.down, m->h, m->y, n, L.ffn_norm));
         } else {
-            TRY(bmm(m, L.wo, m->att, m->y, n, EPI_STORE));
+            TRY(bmm(m, L.wo, m->att, m->y, n, EPI_STORE, f32x));
             TRY(ew_launch(EW_ADD, m->x, m->y, m->x, 0.f, (long)n * d, m->st));
             TRY(rmsnorm_launch(m->x, L.ffn_norm, m->xn, d, n, d, c.rms_eps, m->st));
-            TRY(bmm(m, L.gu, m->xn, m->h, n, EPI_SILU_MUL));
-            TRY(bmm(m, L.down, m->h, m->y, n, EPI_STORE));
+            TRY(bmm(m, L.gu, m->xn, m->h, n, EPI_SILU_MUL, f32x));
+            TRY(bmm(m, L.down, m->h, m->y, n, EPI_STORE, f32x));
             TRY(ew_launch(EW_ADD, m->x, m->y, m->x, 0.f, (long)n * d, m->st));
         }
     }
@@ -1352,7 +1369,7 @@ int run_batch_step(atlas_model* m, int n, const std::vector<int>& slots, bool lo
 // the most prompt rows one step of this model takes
 int prefill_cap(const atlas_model* m) {
     if (!m->fused) return 1;
-    if (!m->big_prefill) return std::min(m->R, kPrefillChunk);
+    if (!m->big_prefill) return m->cfg.post_norm ? std::min(m->R, kPrefillChunk) : 1;
     return std::min(m->R, kPrefillLib);
 }
 
@@ -1441,11 +1458,11 @@ ATLAS_API atlas_model* atlas_model_create(const atlas_model_config* cfg) {
     m->kvd = c.n_kv_heads * hd;
     m->qkv_rows = c.d_model + 2 * m->kvd;
     m->B = c.max_batch < 1 ? 1 : c.max_batch;
-    // big prompt chunks: the fused (post-norm) step, every GEMM inner
+    // big prompt chunks: the fused step, every GEMM inner
     // dimension (d_model, n_heads * head_dim, ffn_hidden) a multiple of the
     // tiled GEMM's 128, and int4 blocks of 32 * 2^j
     const int i4_cpb = fmt == WF_I4 && c.int4_block > 0 ? c.int4_block / 32 : 1;
-    m->big_prefill = (i4_cpb & (i4_cpb - 1)) == 0 && c.post_norm &&
+    m->big_prefill = (i4_cpb & (i4_cpb - 1)) == 0 &&
                      attn_fused_supported(c.n_heads, c.n_kv_heads, hd) &&
                      attn_rows_fit(c.max_seq, c.n_kv_heads, hd) && c.d_model % 128 == 0 &&
                      (c.n_heads * hd) % 128 == 0 && c.ffn_hidden % 128 == 0;
@@ -1553,7 +1570,7 @@ ATLAS_API atlas_model* atlas_model_create(const atlas_model_config* cfg) {
         // initialise its kernel host, then crash, and the cause is not
         // known.  Without a library context the tiled kernel serves every
         // prompt chunk, as it serves int4.
-        if (m->big_prefill && (fmt == WF_BF16 || fmt == WF_I8) && prompt_blas_opt_in()) {
+        if (m->big_prefill && c.post_norm && (fmt == WF_BF16 || fmt == WF_I8) && prompt_blas_opt_in()) {
             int max_m = 0, max_k = 0;
             for (const auto& sh : shapes) {
                 max_m = std::max(max_m, sh[0]);
@@ -1567,11 +1584,17 @@ ATLAS_API atlas_model* atlas_model_create(const atlas_model_config* cfg) {
 
         }
     }
-    // fused step: post-norm model whose attention shape the fused kernel
-    // covers and whose GEMVs take the aligned fast path (d % 32 == 0)
-    m->fused = c.post_norm && attn_fused_supported(c.n_heads, c.n_kv_heads, hd) &&
+    // fused step: a model whose attention shape the fused kernel covers and
+    // whose GEMVs take the aligned fast path (d % 32 == 0)
+    m->fused = attn_fused_supported(c.n_heads, c.n_kv_heads, hd) &&
                attn_rows_fit(c.max_seq, c.n_kv_heads, hd) && d % 32 == 0 &&
                c.ffn_hidden % 32 == 0;
+    if (!c.post_norm)          // the norm of the sum in the prologues of QKV, gate/up and the lm_head
+        for (const DevMat* w : {&m->L[0].qkv, &m->L[0].gu, &m->lm_head}) {
+            GemvArgs a = pro_args(*w, m->xb, m->logits, PRO_ADDNORM, m->y2, m->final_norm, c.rms_eps, m->x);
+            a.epi = w == &m->L[0].gu ? EPI_SILU_MUL : EPI_STORE;
+            m->fused = m->fused && gemv_n2_ok(a);
+        }
     // split partials: the fused kernel's B x n_heads x attn_splits, the
     // long-context step's n_heads x attn_splits_long, or the long-context
     // batch step's n x n_heads x attn_splits_batch[n]
@@ -2127,7 +2150,8 @@ ATLAS_API int atlas_model_bench_gemv(atlas_model* m, int iters, int which, float
             LayerW& L = m->L[li];
             if (qkv_set) {
                 if (m->fused)
-                    TRY(gemv_launch(pro_args(L.qkv, m->xb, m->qkv, PRO_RESNORM, m->y2, L.ffn_norm, eps, m->x), m->st));
+                    TRY(gemv_launch(pro_args(L.qkv, m->xb, m->qkv, m->cfg.post_norm ? PRO_RESNORM : PRO_ADDNORM,
+                                             m->y2, L.ffn_norm, eps, m->x), m->st));
                 else
                     TRY(gemv(m, L.qkv, m->x, m->qkv, EPI_STORE));
             }
@@ -2146,7 +2170,9 @@ ATLAS_API int atlas_model_bench_gemv(atlas_model* m, int iters, int which, float
                 GemvArgs h = pro_args(m->lm_head, m->xb, m->logits, PRO_RESNORM_NORM, m->y2,
                                       m->L.back().ffn_norm, eps, nullptr);
                 h.pro_w2 = m->final_norm;
-                if (!gemv_resnorm_norm_ok(h))
+                if (!m->cfg.post_norm)
+                    h = pro_args(m->lm_head, m->xb, m->logits, PRO_ADDNORM, m->y2, m->final_norm, eps, nullptr);
+                else if (!gemv_n2_ok(h))
                     h = pro_args(m->lm_head, m->xb, m->logits, PRO_RMSNORM, nullptr, m->final_norm,
                                  eps, m->xn);
                 TRY(gemv_launch(h, m->st));

@@ -96,8 +96,13 @@ __device__ __forceinline__ float chunk_dot(const u32x4 w, const f32x4* __restric
 // PRO_RESNORM / PRO_RMSNORM follow rmsnorm_inplace (crates/atlas-model/src/
 // lib.rs:335-342): inv = 1/sqrt(sum(v^2)/n + eps), v*inv*w, and the post-norm
 // residual x + normed (lib.rs:985-993); PRO_SILU is FeedForward's
-// silu(gate) * up (lib.rs:918-921) over interleaved (gate, up) pairs.
+// silu(gate) * up (lib.rs:918-921) over interleaved (gate, up) pairs;
+// PRO_ADDNORM is the pre-norm block's residual add and the norm of the sum
+// (lib.rs:994-1005).  It and PRO_RESNORM_NORM are compiled into instances of
+// their own (N2): in the others the extra branch cost the int4 kernel 1%.
 // ---------------------------------------------------------------------------
+static bool gemv_n2(int pro) { return pro == PRO_RESNORM_NORM || pro == PRO_ADDNORM; }
+
 template <int NW>
 __device__ __forceinline__ float block_sum(float v, float* red) {
     v = wave_sum(v);
@@ -130,7 +135,8 @@ __device__ __forceinline__ void stage_regs_issue(const GemvArgs& a, XRegs<PPT>& 
     const f32x4* yin = reinterpret_cast<const f32x4*>(a.pro_y);
     const f32x4* win = reinterpret_cast<const f32x4*>(a.pro_w);
     const bool norm2 = N2 && a.pro == PRO_RESNORM_NORM;
-    const bool res = a.pro == PRO_RESNORM || norm2, norm = res || a.pro == PRO_RMSNORM;
+    const bool res = a.pro == PRO_RESNORM || norm2 || (N2 && a.pro == PRO_ADDNORM);
+    const bool norm = res || a.pro == PRO_RMSNORM;
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
         const int p = threadIdx.x + NT * j;
@@ -150,7 +156,8 @@ __device__ __forceinline__ void stage_regs_issue(const GemvArgs& a, XRegs<PPT>& 
 template <int PPT, int NT = 256, bool N2 = false>
 __device__ __forceinline__ void stage_regs_issue_buf(const GemvArgs& a, XRegs<PPT>& r, int K) {
     const bool norm2 = N2 && a.pro == PRO_RESNORM_NORM;
-    const bool res = a.pro == PRO_RESNORM || norm2, norm = res || a.pro == PRO_RMSNORM;
+    const bool res = a.pro == PRO_RESNORM || norm2 || (N2 && a.pro == PRO_ADDNORM);
+    const bool norm = res || a.pro == PRO_RMSNORM;
     const __amdgpu_buffer_rsrc_t xb =
         __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(a.x), (short)0, K * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t yb = __builtin_amdgcn_make_buffer_rsrc(
@@ -172,7 +179,14 @@ __device__ __forceinline__ void stage_regs_finish(const GemvArgs& a, XRegs<PPT>&
     __shared__ float red[NT / 64], red2[NT / 64];
     const int np = K >> 2;
     const bool norm2 = N2 && a.pro == PRO_RESNORM_NORM;
-    const bool res = a.pro == PRO_RESNORM || norm2, norm = res || a.pro == PRO_RMSNORM;
+    const bool add = N2 && a.pro == PRO_ADDNORM;
+    const bool res = a.pro == PRO_RESNORM || norm2, norm = res || add || a.pro == PRO_RMSNORM;
+    if constexpr (N2) {
+        if (add) {
+#pragma unroll
+            for (int j = 0; j < PPT; ++j) r.x[j] = r.x[j] + r.y[j];
+        }
+    }
     const f32x4 (&xv)[PPT] = r.x;
     const f32x4 (&yv)[PPT] = r.y;
     const f32x4 (&wv)[PPT] = r.w;
@@ -234,7 +248,7 @@ __device__ __forceinline__ void stage_regs_finish(const GemvArgs& a, XRegs<PPT>&
         if (p < np) {
             if constexpr (N2) xs[SWZ ? xpad(p) : p] = norm2 ? (v[j] * inv2) * w2[j] : v[j];
             else xs[SWZ ? xpad(p) : p] = v[j];
-            if (write_out) reinterpret_cast<f32x4*>(a.pro_out)[p] = v[j];
+            if (write_out) reinterpret_cast<f32x4*>(a.pro_out)[p] = add ? xv[j] : v[j];
         }
     }
 }
@@ -280,13 +294,14 @@ __device__ __forceinline__ void stage_x_loop(const GemvArgs& a, f32x4* xs, int K
     const int np = K >> 2;
     const f32x4* xin = reinterpret_cast<const f32x4*>(a.x);
     const bool norm2 = N2 && a.pro == PRO_RESNORM_NORM;
-    const bool res = a.pro == PRO_RESNORM || norm2;
+    const bool res = a.pro == PRO_RESNORM || norm2, add = N2 && a.pro == PRO_ADDNORM;
     float inv = 1.0f;
-    if (res || a.pro == PRO_RMSNORM) {
+    if (res || add || a.pro == PRO_RMSNORM) {
         const f32x4* v = reinterpret_cast<const f32x4*>(res ? a.pro_y : a.x);
         float ss = 0.f;
         for (int p = threadIdx.x; p < np; p += NT) {
-            const f32x4 t = v[p];
+            f32x4 t = v[p];
+            if (add) t = t + reinterpret_cast<const f32x4*>(a.pro_y)[p];
             ss += t.x * t.x;
             ss += t.y * t.y;
             ss += t.z * t.z;
@@ -295,12 +310,17 @@ __device__ __forceinline__ void stage_x_loop(const GemvArgs& a, f32x4* xs, int K
         ss = block_sum<NT / 64>(ss, red);
         inv = 1.0f / sqrtf(ss / (float)K + a.pro_eps);
     }
-    const bool write_out = a.pro_out && blockIdx.x == 0 && (res || a.pro == PRO_RMSNORM);
+    const bool write_out = a.pro_out && blockIdx.x == 0 && (res || add || a.pro == PRO_RMSNORM);
     float ss2 = 0.f;
     for (int p = threadIdx.x; p < np; p += NT) {
         f32x4 r;
         if (a.pro == PRO_X) {
             r = xin[p];
+        } else if (add) {
+            const f32x4 h = xin[p] + reinterpret_cast<const f32x4*>(a.pro_y)[p];
+            xs[SWZ ? xpad(p) : p] = (h * inv) * reinterpret_cast<const f32x4*>(a.pro_w)[p];
+            if (write_out) reinterpret_cast<f32x4*>(a.pro_out)[p] = h;
+            continue;
         } else if (res) {
             const f32x4 yi = reinterpret_cast<const f32x4*>(a.pro_y)[p];
             const f32x4 wi = reinterpret_cast<const f32x4*>(a.pro_w)[p];
@@ -1221,7 +1241,7 @@ static const void* v4_kernel(int fmt, int rows, int unroll, int nw, bool n2) {
     return nullptr;
 }
 
-bool gemv_resnorm_norm_ok(const GemvArgs& a_in) {
+bool gemv_n2_ok(const GemvArgs& a_in) {
     GemvArgs a = a_in;
     gemv_fill_int4_index(a);
     const uintptr_t align = (uintptr_t)a.w | (uintptr_t)a.x | (uintptr_t)a.pro_y |
@@ -1239,7 +1259,7 @@ int gemv_waves(const GemvArgs& a_in) {
     gemv_fill_int4_index(a);
     const N1Shape v4 = v4_shape(a.fmt, a.M, a.K, a.epi);
     if (v4_ok(a, v4.unroll)) {
-        const void* kern = v4_kernel(a.fmt, v4.rows, v4.unroll, v4.nw, a.pro == PRO_RESNORM_NORM);
+        const void* kern = v4_kernel(a.fmt, v4.rows, v4.unroll, v4.nw, gemv_n2(a.pro));
         return kern ? v4.nw * n1_blocks(kern, a.M, v4_lds_bytes(a.fmt, a.K, v4.unroll),
                                         n1_group_rows(a, v4.rows), v4.bpc, v4.nw)
                     : 0;
@@ -1271,7 +1291,8 @@ int gemv_launch(const GemvArgs& a_in, hipStream_t st) {
     if (a.M == 0) return ATLAS_OK;
     ATLAS_REQUIRE(a.w && a.y, "gemv: null pointer");
     ATLAS_REQUIRE(a.pro == PRO_SILU || a.x, "gemv: null x");
-    ATLAS_REQUIRE(a.pro != PRO_RESNORM || (a.pro_y && a.pro_w), "gemv: residual norm needs y and w");
+    ATLAS_REQUIRE((a.pro != PRO_RESNORM && a.pro != PRO_ADDNORM) || (a.pro_y && a.pro_w),
+                  "gemv: residual norm needs y and w");
     ATLAS_REQUIRE(a.pro != PRO_RMSNORM || a.pro_w, "gemv: rmsnorm prologue needs w");
     ATLAS_REQUIRE(a.pro != PRO_RESNORM_NORM || (a.pro_y && a.pro_w && a.pro_w2),
                   "gemv: residual + final norm prologue needs y, w and w2");
@@ -1296,13 +1317,13 @@ int gemv_launch(const GemvArgs& a_in, hipStream_t st) {
         if (v4_ok(a, v4.unroll)) {
 #define ATLAS_V4(F, R, U, W)                                                          \
             if (a.fmt == F && v4.rows == R && v4.unroll == U && v4.nw == W)                 \
-                return a.pro == PRO_RESNORM_NORM ? launch_v4<F, R, U, W, true>(a, st, v4.bpc) \
-                                                 : launch_v4<F, R, U, W, false>(a, st, v4.bpc);
+                return gemv_n2(a.pro) ? launch_v4<F, R, U, W, true>(a, st, v4.bpc) \
+                                      : launch_v4<F, R, U, W, false>(a, st, v4.bpc);
             ATLAS_V4_LIST(ATLAS_V4)
 #undef ATLAS_V4
         }
-        ATLAS_REQUIRE(a.pro != PRO_RESNORM_NORM,
-                      "gemv: the residual + final norm prologue needs the decode kernel's shapes");
+        ATLAS_REQUIRE(!gemv_n2(a.pro),
+                      "gemv: the residual + norm of the sum prologues need the decode kernel's shapes");
         const N1Shape sh = n1_shape(a.fmt, a.K, a.epi);
 #define ATLAS_N1(F, R, U) \
         if (a.fmt == F && sh.rows == R && sh.unroll == U) return launch_n1<F, R, U>(a, st, sh.bpc);

@@ -11,13 +11,17 @@ __device__ __forceinline__ uint32_t bf16_hi2(float a, float b) {
     return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
 
+// two floats rounded to nearest even, a low
+__device__ __forceinline__ uint32_t bf16_rne2(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 v = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(uint32_t, v);
+}
+
 // the remainders of two floats' truncations, rounded to nearest even, a low
 __device__ __forceinline__ uint32_t bf16_lo2(float a, float b) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const float ra = a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
-    const float rb = b - __uint_as_float(__float_as_uint(b) & 0xFFFF0000u);
-    const bf16x2 v = {(__bf16)ra, (__bf16)rb};
-    return __builtin_bit_cast(uint32_t, v);
+    return bf16_rne2(a - __uint_as_float(__float_as_uint(a) & 0xFFFF0000u),
+                     b - __uint_as_float(__float_as_uint(b) & 0xFFFF0000u));
 }
 
 // two f32 with <= 8 significant bits -> packed bf16 pair (a low), exact

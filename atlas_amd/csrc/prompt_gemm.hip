@@ -80,19 +80,37 @@ __device__ __forceinline__ void sync_stage() {
 template <int FMT>
 using PgRaw = std::conditional_t<FMT == WF_BF16, u32x4, std::conditional_t<FMT == WF_I8, u32x2, uint32_t>>;
 
-// hi and lo operands of 8 activations (int4: in the order the nibble masks give)
-template <int FMT>
-__device__ __forceinline__ void pg_split(const f32x4 p, const f32x4 q, bf16x8& hi, bf16x8& lo) {
-    u32x4 h, l;
+// the bf16 parts of 8 activations (int4: in the order the nibble masks give).
+// NS = 2: hi (truncation) and the rounded remainder; NS = 3: two truncations and
+// the rest, x exactly (8 + 8 + 8 bits).
+// The matrix cores round an f32 sum down, which shifts every result by about
+// -1e-7 of their size: little beside the 5e-6 of two parts, but at three the
+// same in every row, so that it adds up through a model (3.3e-6 of a 1000-token
+// prompt's logits against 1.5e-6).  So with three parts every other k step
+// multiplies -x and its sum is subtracted (flip, the sign bit): what one rounds
+// down the next rounds up.
+template <int FMT, int NS>
+__device__ __forceinline__ void pg_split(const f32x4 p, const f32x4 q, uint32_t flip, bf16x8 (&part)[NS]) {
+    float e[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+    if constexpr (NS == 3)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[i] = __uint_as_float(__float_as_uint(e[i]) ^ flip);
     if constexpr (FMT == WF_I4) {
-        h = u32x4{bf16_hi2(p.y, q.y), bf16_hi2(p.x, q.x), bf16_hi2(p.w, q.w), bf16_hi2(p.z, q.z)};
-        l = u32x4{bf16_lo2(p.y, q.y), bf16_lo2(p.x, q.x), bf16_lo2(p.w, q.w), bf16_lo2(p.z, q.z)};
-    } else {
-        h = u32x4{bf16_hi2(p.x, p.y), bf16_hi2(p.z, p.w), bf16_hi2(q.x, q.y), bf16_hi2(q.z, q.w)};
-        l = u32x4{bf16_lo2(p.x, p.y), bf16_lo2(p.z, p.w), bf16_lo2(q.x, q.y), bf16_lo2(q.z, q.w)};
+        const float o[8] = {p.y, q.y, p.x, q.x, p.w, q.w, p.z, q.z};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[i] = o[i];
     }
-    hi = __builtin_bit_cast(bf16x8, h);
-    lo = __builtin_bit_cast(bf16x8, l);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        u32x4 h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            h[i] = s + 1 < NS ? bf16_hi2(e[2 * i], e[2 * i + 1]) : bf16_rne2(e[2 * i], e[2 * i + 1]);
+        if (s + 1 < NS)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) e[i] -= __uint_as_float(__float_as_uint(e[i]) & 0xFFFF0000u);
+        part[s] = __builtin_bit_cast(bf16x8, h);
+    }
 }
 
 // 8 weights as a bf16 operand; nib: 0x00780078 in a vector register (one
@@ -151,7 +169,7 @@ struct PgShape {
     static constexpr int BYTES = X_OFS + XR * X_BYTES;
 };
 
-template <int FMT, int WM, int WN, int MF, int NF, int VW>
+template <int FMT, int WM, int WN, int MF, int NF, int VW, int NS>
 __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, float* __restrict__ partial,
                                                                   int steps_per_split, int cpb_shift,
                                                                   int m_tiles, int n_tiles) {
@@ -249,7 +267,9 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
         x0[j] = *reinterpret_cast<const f32x4*>(st + xofs0 + j * 2048);
         x1[j] = *reinterpret_cast<const f32x4*>(st + xofs1 + j * 2048);
     };
-    auto split_x = [&](int j, bf16x8& hi, bf16x8& lo) { pg_split<FMT>(x0[j], x1[j], hi, lo); };
+    // (three parts: odd steps with the sign turned)
+    auto flip = [&](int s) { return (uint32_t)(s & 1) << 31; };
+    auto split_x = [&](int j, uint32_t f, bf16x8 (&part)[NS]) { pg_split<FMT, NS>(x0[j], x1[j], f, part); };
     uint32_t nib = 0x00780078u;
     if constexpr (FMT == WF_I4) asm("" : "+v"(nib));
     auto conv_w = [&](int i) {
@@ -269,40 +289,61 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
 
     // activation tile j against every weight tile; last: each weight tile's
     // registers take the next step's tile as soon as it is done
-    auto mfma_group = [&](bf16x8 xh, bf16x8 xl, int j, const uint8_t* wst, int q, bool last) {
+    auto mfma_group = [&](const bf16x8 (&xp)[NS], int j, float sgn, const uint8_t* wst, int q, bool last) {
         if constexpr (FMT == WF_I4) {
             const bf16x8 off = __builtin_bit_cast(bf16x8, neg24);
-            f32x4 d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, off, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, off, d0, 0, 0, 0);
+            f32x4 d0 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < NS; ++s) d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[s], off, d0, 0, 0, 0);
             constexpr int H = MF / 2;
 #pragma unroll
             for (int h = 0; h < MF; h += H) {
                 f32x4 d[H];
 #pragma unroll
-                for (int i = 0; i < H; ++i) d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, w_op(h + i), d0, 0, 0, 0);
+                for (int s = 0; s < NS; ++s)
 #pragma unroll
-                for (int i = 0; i < H; ++i) {
-                    d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, w_op(h + i), d[i], 0, 0, 0);
-                    if (last) conv_w(h + i);
-                }
+                    for (int i = 0; i < H; ++i) {
+                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[s], w_op(h + i), s ? d[i] : d0, 0, 0, 0);
+                        if (last && s + 1 == NS) conv_w(h + i);
+                    }
 #pragma unroll
                 for (int i = 0; i < H; ++i) acc[j][h + i] += d[i] * sc[h + i];
             }
             if (last)
 #pragma unroll
                 for (int i = 0; i < MF; ++i) sc[i] = scn[i];
+        } else if constexpr (NS == 3) {
+            // small parts first; each step's sum joins the running one by a
+            // rounded addition
+            constexpr int H = MF / 2;
+#pragma unroll
+            for (int h = 0; h < MF; h += H) {
+                f32x4 d[H];
+#pragma unroll
+                for (int s = NS - 1; s >= 0; --s)
+#pragma unroll
+                    for (int i = 0; i < H; ++i) {
+                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            xp[s], w_op(h + i), s == NS - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[i], 0, 0, 0);
+                        if (last && s == 0) {
+                            if constexpr (FMT == WF_BF16) read_w(wst, q, h + i);
+                            else conv_w(h + i);
+                        }
+                    }
+#pragma unroll
+                for (int i = 0; i < H; ++i) acc[j][h + i] += d[i] * sgn;
+            }
         } else {
 #pragma unroll
-            for (int i = 0; i < MF; ++i)
-                acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, w_op(i), acc[j][i], 0, 0, 0);
+            for (int s = 0; s < NS; ++s)
 #pragma unroll
-            for (int i = 0; i < MF; ++i) {
-                acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, w_op(i), acc[j][i], 0, 0, 0);
-                if (last) {
-                    if constexpr (FMT == WF_BF16) read_w(wst, q, i);
-                    else conv_w(i);
+                for (int i = 0; i < MF; ++i) {
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[s], w_op(i), acc[j][i], 0, 0, 0);
+                    if (last && s + 1 == NS) {
+                        if constexpr (FMT == WF_BF16) read_w(wst, q, i);
+                        else conv_w(i);
+                    }
                 }
-            }
         }
     };
 
@@ -338,8 +379,8 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
 #pragma unroll
         for (int i = 0; i < MF; ++i) sc[i] = scn[i];
     }
-    bf16x8 xh, xl;
-    split_x(0, xh, xl);
+    bf16x8 xp[NS];
+    split_x(0, 0, xp);
 
     // One k step s (step q of its weight unit): its fragments are in registers
     // (tile 0's split done), and step s + 1 has landed at the barrier.
@@ -347,7 +388,7 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
     auto compute = [&](int s, int q) {
         const uint8_t *wst = w_unit(s + 1), *xst = x_slot(s + 1);
         const int qn = (q + 1) % S::KU;
-        bf16x8 yh, yl;
+        bf16x8 yp[NS];
         __builtin_amdgcn_sched_barrier(0);
         read_x(xst, 0);
 #pragma unroll
@@ -357,14 +398,14 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
                 for (int i = j * WPG; i < min(MF, (j + 1) * WPG); ++i) read_w(wst, qn, i);
             }
             if (j + 1 < NF) {
-                split_x(j + 1, yh, yl);
+                split_x(j + 1, flip(s), yp);
                 read_x(xst, j + 1);
             } else {
-                split_x(0, yh, yl);
+                split_x(0, flip(s + 1), yp);
             }
-            mfma_group(xh, xl, j, wst, qn, j + 1 == NF);
-            xh = yh;
-            xl = yl;
+            mfma_group(xp, j, (s & 1) ? -1.0f : 1.0f, wst, qn, j + 1 == NF);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) xp[s] = yp[s];
         }
     };
     // At the barrier of step s the slots of step s - 1 are free (every wave
@@ -463,7 +504,7 @@ struct FrShape {
     static constexpr int BYTES = UR * UNIT > RED ? UR * UNIT : RED;
 };
 
-template <int FMT, int MF, int NF, int VW>
+template <int FMT, int MF, int NF, int VW, int NS>
 __global__ __launch_bounds__(512) void few_rows_gemm_kernel(GemvArgs a, float* __restrict__ partial,
                                                              int units_per_split, int cpb_shift) {
     using S = FrShape<FMT, MF, NF, VW>;
@@ -555,34 +596,36 @@ __global__ __launch_bounds__(512) void few_rows_gemm_kernel(GemvArgs a, float* _
             w[i] = *reinterpret_cast<const PgRaw<FMT>*>(st + wofs + i * 16 * S::RB);
             if constexpr (FMT == WF_I4) sc[i] = *reinterpret_cast<const float*>(st + sofs + i * 64);
         }
-        bf16x8 xh[NF], xl[NF];
+        bf16x8 xp[NF][NS];
+        const uint32_t flip = (uint32_t)(kg & 1) << 31;             // the step is KG u + kg
+        const float sgn = (kg & 1) ? -1.0f : 1.0f;
         f32x4 d0[FMT == WF_I4 ? NF : 1];
 #pragma unroll
         for (int j = 0; j < NF; ++j) {
-            pg_split<FMT>(x0[j], x1[j], xh[j], xl[j]);
+            pg_split<FMT, NS>(x0[j], x1[j], flip, xp[j]);
             if constexpr (FMT == WF_I4) {
-                d0[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh[j], off, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                d0[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl[j], off, d0[j], 0, 0, 0);
+                d0[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < NS; ++s) d0[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[j][s], off, d0[j], 0, 0, 0);
             }
         }
 #pragma unroll
         for (int i = 0; i < MF; ++i) {
             const bf16x8 b = pg_operand<FMT>(w[i], nib);
-            if constexpr (FMT == WF_I4) {
-                f32x4 d[NF];
+            f32x4 d[NF];
 #pragma unroll
-                for (int j = 0; j < NF; ++j) d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh[j], b, d0[j], 0, 0, 0);
+            for (int j = 0; j < NF; ++j)
+                d[j] = FMT == WF_I4 ? d0[FMT == WF_I4 ? j : 0] : NS == 3 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[j][i];
 #pragma unroll
-                for (int j = 0; j < NF; ++j) d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl[j], b, d[j], 0, 0, 0);
-#pragma unroll
-                for (int j = 0; j < NF; ++j) acc[j][i] += d[j] * sc[i];
-            } else {
+            for (int s = 0; s < NS; ++s)                       // (three parts: the small ones first)
 #pragma unroll
                 for (int j = 0; j < NF; ++j)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh[j], b, acc[j][i], 0, 0, 0);
+                    d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[j][NS == 3 ? 2 - s : s], b, d[j], 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < NF; ++j)
-                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl[j], b, acc[j][i], 0, 0, 0);
+            for (int j = 0; j < NF; ++j) {
+                if constexpr (FMT == WF_I4) acc[j][i] += d[j] * sc[i];
+                else if constexpr (NS == 3) acc[j][i] += d[j] * sgn;
+                else acc[j][i] = d[j];
             }
         }
     };
@@ -692,56 +735,68 @@ static PgPlan pg_plan(int fmt, int M, int N, int K, bool split_ok) {
     return best;
 }
 
-template <int FMT, int WM, int WN, int MF, int NF, int VW>
+template <int FMT, int WM, int WN, int MF, int NF, int VW = 16>
 static void pg_go(const GemvArgs& a, const PgPlan& p, float* partial, int cpb_shift, hipStream_t st) {
     using S = PgShape<FMT, WM, WN, MF, NF, VW>;
     static_assert(S::BYTES <= 160 * 1024, "LDS of a CU");
     const int mt = (a.M + S::BM - 1) / S::BM, nt = (a.N + S::BN - 1) / S::BN;
-    hipLaunchKernelGGL((prompt_gemm_kernel<FMT, WM, WN, MF, NF, VW>), dim3((mt + 7) / 8 * 8 * nt, p.splits),
-                       dim3(S::THREADS), S::BYTES, st, a, partial, p.steps, cpb_shift, mt, nt);
+    const dim3 grid((mt + 7) / 8 * 8 * nt, p.splits);
+    if constexpr (FMT != WF_I4) {
+        if (a.f32x) {
+            hipLaunchKernelGGL((prompt_gemm_kernel<FMT, WM, WN, MF, NF, VW, 3>), grid, dim3(S::THREADS), S::BYTES,
+                               st, a, partial, p.steps, cpb_shift, mt, nt);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((prompt_gemm_kernel<FMT, WM, WN, MF, NF, VW, 2>), grid, dim3(S::THREADS), S::BYTES, st, a,
+                       partial, p.steps, cpb_shift, mt, nt);
 }
 
-template <int FMT, int MF, int NF, int VW>
+template <int FMT, int MF, int NF, int VW = 16>
 static void fr_go(const GemvArgs& a, const PgPlan& p, float* partial, int cpb_shift, hipStream_t st) {
     using S = FrShape<FMT, MF, NF, VW>;
     static_assert(S::BYTES <= 160 * 1024, "LDS of a CU");
-    hipLaunchKernelGGL((few_rows_gemm_kernel<FMT, MF, NF, VW>),
-                       dim3((a.M + S::BM - 1) / S::BM, p.splits, (a.N + S::BN - 1) / S::BN), dim3(S::THREADS),
-                       S::BYTES, st, a, partial, p.steps, cpb_shift);
+    const dim3 grid((a.M + S::BM - 1) / S::BM, p.splits, (a.N + S::BN - 1) / S::BN);
+    if constexpr (FMT != WF_I4) {
+        if (a.f32x) {
+            hipLaunchKernelGGL((few_rows_gemm_kernel<FMT, MF, NF, VW, 3>), grid, dim3(S::THREADS), S::BYTES, st, a,
+                               partial, p.steps, cpb_shift);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((few_rows_gemm_kernel<FMT, MF, NF, VW, 2>), grid, dim3(S::THREADS), S::BYTES, st, a, partial,
+                       p.steps, cpb_shift);
 }
 
 // 16-byte loads need 16-byte aligned weight rows; others (int8 from 8, int4
 // from 4 bytes up) load 4 bytes per lane, in one tile of each kind
 template <int FMT>
 static void pg_launch(const GemvArgs& a, const PgPlan& p, float* partial, int sh, hipStream_t st) {
-    const bool few = p.few;
     const int nf = fr_nf(a.N);
     if constexpr (FMT != WF_BF16) {
         if (((uintptr_t)a.w | (uintptr_t)a.ldw) & 15) {
-            if (!few) pg_go<FMT, 2, 4, 4, 2, 4>(a, p, partial, sh, st);
+            if (!p.few) pg_go<FMT, 2, 4, 4, 2, 4>(a, p, partial, sh, st);
             else if (nf == 1) fr_go<FMT, 2, 1, 4>(a, p, partial, sh, st);
             else if (nf == 2) fr_go<FMT, 2, 2, 4>(a, p, partial, sh, st);
             else fr_go<FMT, 2, 4, 4>(a, p, partial, sh, st);
             return;
         }
     }
-    if (few) {
-        if (p.tile == 2) {
-            if (nf == 1) fr_go<FMT, 2, 1, 16>(a, p, partial, sh, st);
-            else if (nf == 2) fr_go<FMT, 2, 2, 16>(a, p, partial, sh, st);
-            else fr_go<FMT, 2, 4, 16>(a, p, partial, sh, st);
-        } else {
-            if (nf == 1) fr_go<FMT, 4, 1, 16>(a, p, partial, sh, st);
-            else if (nf == 2) fr_go<FMT, 4, 2, 16>(a, p, partial, sh, st);
-            else fr_go<FMT, 4, 4, 16>(a, p, partial, sh, st);
+    if (p.few && p.tile == 2) {
+        if (nf == 1) fr_go<FMT, 2, 1>(a, p, partial, sh, st);
+        else if (nf == 2) fr_go<FMT, 2, 2>(a, p, partial, sh, st);
+        else fr_go<FMT, 2, 4>(a, p, partial, sh, st);
+    } else if (p.few) {
+        if (nf == 1) fr_go<FMT, 4, 1>(a, p, partial, sh, st);
+        else if (nf == 2) fr_go<FMT, 4, 2>(a, p, partial, sh, st);
+        else fr_go<FMT, 4, 4>(a, p, partial, sh, st);
+    } else {
+        switch (p.tile) {
+        case PG_256x128: pg_go<FMT, 2, 4, 8, 2>(a, p, partial, sh, st); break;
+        case PG_192x128: pg_go<FMT, 2, 4, 6, 2>(a, p, partial, sh, st); break;
+        case PG_128x128: pg_go<FMT, 2, 4, 4, 2>(a, p, partial, sh, st); break;
+        default: pg_go<FMT, 4, 2, 4, 2>(a, p, partial, sh, st); break;
         }
-        return;
-    }
-    switch (p.tile) {
-    case PG_256x128: pg_go<FMT, 2, 4, 8, 2, 16>(a, p, partial, sh, st); break;
-    case PG_192x128: pg_go<FMT, 2, 4, 6, 2, 16>(a, p, partial, sh, st); break;
-    case PG_128x128: pg_go<FMT, 2, 4, 4, 2, 16>(a, p, partial, sh, st); break;
-    default: pg_go<FMT, 4, 2, 4, 2, 16>(a, p, partial, sh, st); break;
     }
 }
 

@@ -1552,11 +1552,12 @@ int skinny_launch(const GemvArgs& a_in, hipStream_t st) {
     GemvArgs a = a_in;
     if (a.defer_splits) *a.defer_splits = 0;
     gemv_fill_int4_index(a);
-    const bool rows_ok = few_rows_pay(a) && a.w && a.x && a.y && gemm_rows_ok(a);
-    if (rows_ok && a.N > 16 && a.blas && (a.fmt == WF_BF16 || (a.fmt == WF_I8 && a.K <= kDigitsMaxK)))
+    const bool rows_ok = (few_rows_pay(a) || a.f32x) && a.w && a.x && a.y && gemm_rows_ok(a);
+    if (rows_ok && a.N > 16 && a.blas && !a.f32x && (a.fmt == WF_BF16 || (a.fmt == WF_I8 && a.K <= kDigitsMaxK)))
         return blas_rows_launch(a.blas, a, st);
     if (rows_ok && gemm_rows_fit(a) && (a.N > 16 || gemv_pitch_ok(a)))
         return gemm_rows_launch(a, rows_need_scratch(a), st);
+    ATLAS_REQUIRE(!a.f32x, "skinny: 24-bit activations need the prompt GEMMs' shapes (M %d K %d)", a.M, a.K);
     if (rows_ok && a.N > 16) {               // rows too long for their offsets: 16 at a time
         for (int n0 = 0; n0 < a.N; n0 += 16) {
             GemvArgs p = a;
