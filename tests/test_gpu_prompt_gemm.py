@@ -61,10 +61,16 @@ def test_prompt_gemm(orc, fmt, n, M, K, block, off, epi):
     got = dy.get().astype(np.float64)
     x64 = x.astype(np.float64)
     ref, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64).T
+    if fmt == "int8":
+        # three digits, where they are taken: 2^-24 of the row's largest element per
+        # product, the sums exact, a few roundings to combine them
+        dig = 2.0**-24 * np.max(np.abs(x64), 1)[:, None] * np.sum(np.abs(w64), 1)[None, :] + 8 * 2.0**-24 * np.abs(ref)
     # x in two bf16 parts: the remainder of an 8-bit truncation rounded to 8 bits,
     # 2^-16 of each product; sums of K products in f32: K/2 roundings of 2^-24
     # (tree or chain, both within K 2^-24 of the magnitudes)
     tol = (2.0**-16 + K * 2.0**-24) * mag
+    if fmt == "int8":
+        tol = np.maximum(tol, dig)
     if fmt == "int4":
         # each step's 32 products run around the offset 24: 33 roundings of
         # sums of at most 32 s |x| per element
@@ -77,3 +83,25 @@ def test_prompt_gemm(orc, fmt, n, M, K, block, off, epi):
         # |silu'| <= 1.1; the epilogue itself rounds a few times
         tol = 1.1 * tg * np.abs(u) + np.abs(g * sg) * tu + 1.1 * tg * tu + 8 * 2.0**-24 * np.abs(ref)
     assert np.all(np.abs(got - ref) <= tol), float(np.max(np.abs(got - ref) / tol))
+
+
+def test_int8_digits_special_rows(orc):
+    # rows with a NaN, an infinity, only zeros, one huge element; the others are
+    # untouched by them
+    n, M, K = 300, 6200, 512
+    print(f"int8 digits special rows n={n} M={M} K={K}", flush=True)
+    rng = np.random.default_rng(5)
+    w = (rng.standard_normal((M, K)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    x[3, 17], x[130, 0], x[131], x[299, 511] = np.nan, np.inf, 0.0, 1e30
+    q, s = orc.int8_quantize(w)
+    w64 = orc.int8_dequantize(q, s).astype(np.float64)
+    dw, ds, dx, dy = Dev(q), Dev(s), Dev(x), Dev(np.full((n, M), 7, np.float32))
+    assert lib().atlas_gemm_skinny_f32(2, dw.ptr, ds.ptr, 0, dx.ptr, dy.ptr, M, n, K) == 0
+    got = dy.get().astype(np.float64)
+    assert np.all(np.isnan(got[3])) and not np.any(np.isfinite(got[130])) and np.all(got[131] == 0)
+    rest = [i for i in range(n) if i not in (3, 130)]
+    ref = x[rest].astype(np.float64) @ w64.T
+    tol = (2.0**-24 * np.max(np.abs(x[rest]).astype(np.float64), 1)[:, None] * np.sum(np.abs(w64), 1)[None, :]
+           + 8 * 2.0**-24 * np.abs(ref))
+    assert np.all(np.abs(got[rest] - ref) <= tol)
