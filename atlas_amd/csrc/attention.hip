@@ -700,7 +700,9 @@ __global__ __launch_bounds__(64 * W) void attn_fused_kernel(AttnFusedArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         pos = __builtin_amdgcn_readfirstlane(pos_v);
     } else {
-        pos = a.pos_dev[seq];
+        // by value for a caller that knows it on the host (one sequence): no
+        // copy of it ahead of the launch, no dependent load inside
+        pos = a.pos_dev ? a.pos_dev[seq] : a.pos;
     }
 
     const int slot = LIVE ? 0 : (a.slot_dev ? a.slot_dev[seq] : 0);
@@ -910,8 +912,9 @@ bool attn_fused_supported(int n_heads, int n_kv, int head_dim) {
 int attn_fused_launch(const AttnFusedArgs& a, int n_splits, int n_seq, hipStream_t st) {
     ATLAS_REQUIRE(attn_fused_supported(a.n_heads, a.n_kv, a.head_dim),
                   "attention: fused path needs head_dim 64/128/256 and group 1/2/4/8");
-    ATLAS_REQUIRE(a.qkv && a.k_cache && a.v_cache && a.out && a.pos_dev && a.cos_tab && a.sin_tab,
+    ATLAS_REQUIRE(a.qkv && a.k_cache && a.v_cache && a.out && a.cos_tab && a.sin_tab,
                   "attention: null pointer");
+    ATLAS_REQUIRE(a.pos_dev || (n_seq == 1 && a.pos >= 0 && !a.rope_row), "attention: position");
     ATLAS_REQUIRE(n_splits == 1 || (a.part_m && a.part_l && a.part_o && a.counters),
                   "attention: split partials missing");
     ATLAS_REQUIRE(n_seq >= 1 && n_splits >= 1, "attention: empty grid");

@@ -52,7 +52,8 @@ struct AttnFusedArgs {
     float* v_cache;
     long slot_stride;
     const int* slot_dev;     // [n_seq] or null (slot 0)
-    const int* pos_dev;      // [n_seq]
+    const int* pos_dev;      // [n_seq], or null: one sequence at pos
+    int pos;
     float* out;              // per sequence [n_heads*hd]
     long out_stride;
     int n_heads, n_kv, head_dim;

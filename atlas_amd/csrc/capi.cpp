@@ -249,20 +249,19 @@ ATLAS_API int atlas_attention_fused_f32(const float* qkv, const float* q_norm,
     const int ctx = (window > 0 && pos + 1 > window) ? window : pos + 1;
     if (n_splits <= 0) n_splits = attn_pick_splits(n_kv, ctx);
     ATLAS_REQUIRE(n_splits <= 1024, "attention_fused: n_splits %d", n_splits);
-    // the calling thread's scratch: position, merge counters (cleared when
-    // grown; the kernel leaves them at zero), split partials
-    void *d_pos = nullptr, *d_cnt = nullptr, *d_part_v = nullptr;
+    // the calling thread's scratch: merge counters (cleared when grown; the
+    // kernel leaves them at zero), split partials.  The position goes by value
+    // (an upload of it ahead of the launch cost 3 us a call).
+    void *d_cnt = nullptr, *d_part_v = nullptr;
     const size_t need = (size_t)n_heads * n_splits * (head_dim + 2) * sizeof(float);
-    int rc = thread_scratch(SCR_FUSED_POS, sizeof(int), &d_pos);
-    if (!rc) rc = thread_scratch(SCR_FUSED_CNT, (size_t)n_kv * sizeof(int), &d_cnt, true);
+    int rc = thread_scratch(SCR_FUSED_CNT, (size_t)n_kv * sizeof(int), &d_cnt, true);
     if (!rc) rc = thread_scratch(SCR_FUSED_PART, need, &d_part_v);
     if (rc) return rc;
     float* d_part = static_cast<float*>(d_part_v);
-    ATLAS_HIP(hipMemcpyAsync(d_pos, &pos, sizeof(int), hipMemcpyHostToDevice, stream()));
     AttnFusedArgs a{};
     a.qkv = qkv; a.qkv_stride = 0; a.q_norm = q_norm; a.k_norm = k_norm; a.qk_eps = qk_eps;
     a.cos_tab = cos_tab; a.sin_tab = sin_tab; a.k_cache = k_cache; a.v_cache = v_cache;
-    a.slot_stride = 0; a.slot_dev = nullptr; a.pos_dev = static_cast<const int*>(d_pos);
+    a.slot_stride = 0; a.slot_dev = nullptr; a.pos_dev = nullptr; a.pos = pos;
     a.out = out; a.out_stride = 0;
     a.n_heads = n_heads; a.n_kv = n_kv; a.head_dim = head_dim; a.scale = scale; a.window = window;
     a.part_m = d_part;

@@ -34,7 +34,6 @@ enum ScratchSlot {
     SCR_ARGMAX,         // argmax per-block keys
     SCR_FUSED_PART,     // atlas_attention_fused_f32 split partials
     SCR_FUSED_CNT,      // ... its merge counters (kept at zero by the kernel)
-    SCR_FUSED_POS,      // ... its position word
     SCR_ATTN_CNT,       // atlas_decode_attention merge counters (kept at zero)
     SCR_DIGITS,         // prompt-GEMM int8 digits of the activations
     SCR_N
