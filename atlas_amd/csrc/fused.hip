@@ -863,6 +863,68 @@ __device__ int sorted_tokens(const uint32_t* hist, int lo, int hi, uint32_t* s) 
     return len;
 }
 
+// f(token, times seen) once per distinct token of hist[lo, hi), each on one
+// thread.  Up to kPairLen tokens every thread compares its own with all (a
+// sort's 36 barrier steps cost 4 us at 200 tokens, the comparisons 0.5).
+constexpr int kPairLen = 256;
+template <class F>
+__device__ void for_distinct(const uint32_t* hist, int lo, int hi, uint32_t* s, F f) {
+    const int tid = threadIdx.x, len = hi - lo;
+    if (len <= kPairLen) {
+        if (tid < kPairLen) s[tid] = tid < len ? hist[lo + tid] : 0xFFFFFFFFu;
+        __syncthreads();
+        if (tid < len) {
+            const uint32_t t = s[tid];
+            int seen = 0, before = 0;
+            for (int j = 0; j < len; ++j) {
+                const int same = s[j] == t;
+                seen += same;
+                before += same && j < tid;
+            }
+            if (!before) f(t, seen);
+        }
+        return;
+    }
+    const int wl = sorted_tokens(hist, lo, hi, s);
+    for (int i = tid; i < wl; i += 1024) {
+        const uint32_t t = s[i];
+        if (i > 0 && s[i - 1] == t) continue;
+        int j = i + 1;
+        while (j < wl && s[j] == t) ++j;
+        f(t, j - i);
+    }
+}
+
+// One wave adding val(0), val(1), ... val(m - 1) one after the other (the
+// reference's order), 64 values in its lanes at a time: a step is a lane read
+// and an add, where a thread walking LDS waits for each value and each exit test.
+// Returns the sum; *first (if asked for) the first i at which hit(running sum),
+// m if there is none.
+template <class V, class H>
+__device__ __forceinline__ float wave_run(int m, V val, H hit, int* first) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63;
+    float acc = 0.0f;
+    for (int b = 0; b < m; b += 64) {
+        const int v = __float_as_int(b + lane < m ? val(b + lane) : 0.0f);
+        float mine = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 64; ++j) {
+            acc += __int_as_float(__builtin_amdgcn_readlane(v, j));
+            mine = lane == j ? acc : mine;
+        }
+        if (first) {
+            const unsigned long long at = __ballot(b + lane < m && hit(mine));
+            if (at) {
+                *first = b + __ffsll((long long)at) - 1;
+                return acc;
+            }
+        }
+    }
+    if (first) *first = m;
+    return acc;
+}
+
 // ---- top_k = 0 with top_p off: the whole vocabulary samples ----------------
 // The reference sums p_i = exp(v_i - max) sequentially in f32, scales them by
 // inv = 1 / sum and takes the first i whose sequential f32 running sum of
@@ -1231,18 +1293,20 @@ __device__ uint32_t sample_all_vocab(float* x, int n, const SampleCfg& c, float 
     return (uint32_t)flag[1];       // n - 1 when no running sum exceeds u
 }
 
+constexpr int kWaveCand = SAMPLE_CAND / 16;     // candidates a wave lists in one scan
+
 __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
 #pragma clang fp contract(off)
     __shared__ uint32_t s_hist[SAMPLE_MAX_HIST];
     __shared__ int s_bins[2048];
     __shared__ int s_idx[SAMPLE_MAX_K];
     __shared__ float s_val[SAMPLE_MAX_K];
-    __shared__ float s_p[SAMPLE_MAX_K];
+    __shared__ __attribute__((aligned(16))) float s_p[SAMPLE_MAX_K];
     __shared__ int s_ord[SAMPLE_MAX_K];
     __shared__ int s_scan[17];
-    __shared__ uint32_t s_ck[SAMPLE_CAND];      // top-k candidates: keys, index order
-    __shared__ int s_ci[SAMPLE_CAND];           // and their indices
-    __shared__ int s_wbase[17];
+    __shared__ __attribute__((aligned(16))) uint32_t s_ck[SAMPLE_CAND];   // top-k candidates: keys, index order
+    __shared__ int s_ci[SAMPLE_CAND];                                     // and their indices
+    __shared__ int s_wbase[18];
     __shared__ float s_red[16];
     __shared__ int s_pick[2];
     __shared__ float s_sum;
@@ -1259,23 +1323,18 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
     __syncthreads();
     // A token seen r times in the window is penalised r times in a row (the
     // reference's loop in history order); distinct tokens are independent, so
-    // one thread per distinct token of the sorted window gives the same values.
+    // one thread per distinct token of the window gives the same values.
     // The host admits windows of at most SAMPLE_MAX_HIST tokens on this path.
     if (c.theta != 1.0f && len > 0) {
         int start = len > c.window ? len - c.window : 0;
         if (len - start > SAMPLE_MAX_HIST) start = len - SAMPLE_MAX_HIST;
-        const int wl = sorted_tokens(a.hist, start, len, s_hist);
-        for (int i = tid; i < wl; i += 1024) {
-            const uint32_t t = s_hist[i];
-            if (i > 0 && s_hist[i - 1] == t) continue;
-            int j = i + 1;
-            while (j < wl && s_hist[j] == t) ++j;
+        for_distinct(a.hist, start, len, s_hist, [&](uint32_t t, int times) {
             if (t < (uint32_t)n) {
                 float v = x[t];
-                for (int r = i; r < j; ++r) v = v > 0.0f ? v / c.theta : v * c.theta;
+                for (int r = 0; r < times; ++r) v = v > 0.0f ? v / c.theta : v * c.theta;
                 x[t] = v;
             }
-        }
+        });
         __syncthreads();
     }
 
@@ -1283,19 +1342,14 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
     // host admits at most SAMPLE_MAX_HIST history entries on this path
     const int hl = len < SAMPLE_MAX_HIST ? len : SAMPLE_MAX_HIST;
     if ((c.freq != 0.0f || c.presence != 0.0f) && hl > 0) {
-        sorted_tokens(a.hist, 0, hl, s_hist);
-        for (int i = tid; i < hl; i += 1024) {
-            const uint32_t t = s_hist[i];
-            if (i > 0 && s_hist[i - 1] == t) continue;
-            int j = i + 1;
-            while (j < hl && s_hist[j] == t) ++j;
+        for_distinct(a.hist, 0, hl, s_hist, [&](uint32_t t, int times) {
             if (t < (uint32_t)n) {
                 float v = x[t];
-                if (c.freq != 0.0f) v -= c.freq * (float)(j - i);
+                if (c.freq != 0.0f) v -= c.freq * (float)times;
                 if (c.presence != 0.0f) v -= c.presence;
                 x[t] = v;
             }
-        }
+        });
         __syncthreads();
     }
 
@@ -1335,83 +1389,153 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
     if (k > SAMPLE_MAX_K) k = SAMPLE_MAX_K;
     if (k > n) k = n;
     const int lane = tid & 63, wv = tid >> 6;
-    // (a) The k-th largest of the 1024 per-thread maxima is a lower bound L of
-    // th: those k maxima are k distinct entries >= it.
-    uint32_t kmax = 0;
-    for (int base = tid; base < n; base += 1024 * 16) {
-        float v[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int i = base + u * 1024;
-            v[u] = x[i < n ? i : n - 1];
-        }
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const uint32_t key = sample_key(v[u] / T);
-            if (base + u * 1024 < n && key > kmax) kmax = key;
-        }
-    }
-    s_hist[tid] = kmax;                          // the penalties are done with s_hist
-    __syncthreads();
-    uint32_t L, th;
+    // Both scans compare logits as they are: v / T never falls as v grows, so
+    // the division is left to the few candidates (at T = inf quotients have no
+    // such order: the general scans below).  One division per entry and scan,
+    // 4 loads in flight and a second scan to write the candidates took 56 us of
+    // this kernel at 100k entries (83 -> 44 us in all at top-k 40, top-p 0.95).
+    int n_cand = SAMPLE_CAND + 1;
+    uint32_t th;
     int need, m;
-    lds_select(s_hist, 1024, k, s_bins, s_pick, &L, &need);
-    // (b) entries with key >= L, counted then written in index order: wave wv
-    // owns a contiguous range and takes 4 x 64 consecutive entries per step
-    const int chunk = ((n + 15) / 16 + 255) & ~255;
-    const int c_lo = wv * chunk < n ? wv * chunk : n;
-    const int c_hi = c_lo + chunk < n ? c_lo + chunk : n;
-    int wcount = 0;
-    for (int b = c_lo; b < c_hi; b += 256) {
-        float v[4];
+    if (T < INFINITY) {
+        // (a) The k-th largest of the 1024 per-thread maxima bounds the k-th
+        // largest entry from below: those k maxima are k distinct entries.
+        uint32_t kmax = 0;
+        for (int base = tid; base < n; base += 1024 * 32) {
+            float v[32];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = b + u * 64 + lane;
-            v[u] = x[i < n ? i : n - 1];
-        }
+            for (int u = 0; u < 32; ++u) {
+                const int i = base + u * 1024;
+                v[u] = x[i < n ? i : n - 1];
+            }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = b + u * 64 + lane;
-            wcount += __popcll(__ballot(i < c_hi && sample_key(v[u] / T) >= L));
+            for (int u = 0; u < 32; ++u) {
+                const uint32_t key = sample_key(v[u]);
+                if (base + u * 1024 < n && key > kmax) kmax = key;
+            }
         }
-    }
-    if (lane == 0) s_wbase[wv] = wcount;
-    __syncthreads();
-    if (tid == 0) {
-        int acc = 0;
-        for (int w = 0; w < 16; ++w) {
-            const int t = s_wbase[w];
-            s_wbase[w] = acc;
-            acc += t;
+        s_hist[tid] = kmax;                      // the penalties are done with s_hist
+        __syncthreads();
+        uint32_t L;
+        lds_select(s_hist, 1024, k, s_bins, s_pick, &L, &need);
+        // the least logit whose quotient is still L's (ties of the quotient are
+        // kept by index, so all of them are candidates): the step below L is
+        // doubled until the quotient falls, then halved
+        const uint32_t Lq = sample_key(sample_unkey(L) / T);
+        uint32_t down = 1;
+        while (down < L && sample_key(sample_unkey(L - down) / T) >= Lq && !(down >> 31)) down <<= 1;
+        uint32_t lo_k = L > down ? L - down : 0, hi_k = L;   // hi_k keeps the quotient
+        while (hi_k - lo_k > 1) {
+            const uint32_t mid = lo_k + (hi_k - lo_k) / 2;
+            if (sample_key(sample_unkey(mid) / T) >= Lq) hi_k = mid;
+            else lo_k = mid;
         }
-        s_wbase[16] = acc;
-    }
-    __syncthreads();
-    const int n_cand = s_wbase[16];
-    if (n_cand <= SAMPLE_CAND) {
-        int pos = s_wbase[wv];
-        for (int b = c_lo; b < c_hi; b += 256) {
-            float v[4];
+        L = lo_k == 0 ? 0 : hi_k;
+        // (b) entries from L up, in index order: wave wv owns a contiguous range
+        // and lists its candidates in its own part of s_ck / s_ci
+        const int chunk = ((n + 15) / 16 + 255) & ~255;
+        const int c_lo = wv * chunk < n ? wv * chunk : n;
+        const int c_hi = c_lo + chunk < n ? c_lo + chunk : n;
+        int wcount = 0;
+        for (int b = c_lo; b < c_hi; b += 1024) {
+            float v[16];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < 16; ++u) {
                 const int i = b + u * 64 + lane;
                 v[u] = x[i < n ? i : n - 1];
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < 16; ++u) {
                 const int i = b + u * 64 + lane;
-                const uint32_t key = sample_key(v[u] / T);
-                const bool in = i < c_hi && key >= L;
+                const bool in = i < c_hi && sample_key(v[u]) >= L;
                 const unsigned long long bal = __ballot(in);
-                if (in) {
-                    const int at = pos + __popcll(bal & ((1ull << lane) - 1));
-                    s_ck[at] = key;
-                    s_ci[at] = i;
+                if (bal) {
+                    const int at = wcount + __popcll(bal & ((1ull << lane) - 1));
+                    if (in && at < kWaveCand) {
+                        s_ck[wv * kWaveCand + at] = sample_key(v[u] / T);
+                        s_ci[wv * kWaveCand + at] = i;
+                    }
+                    wcount += __popcll(bal);
                 }
-                pos += __popcll(bal);
+            }
+        }
+        if (lane == 0) s_wbase[wv] = wcount;
+        __syncthreads();
+        if (tid == 0) {
+            int acc = 0, most = 0;
+            for (int w = 0; w < 16; ++w) {
+                const int t = s_wbase[w];
+                s_wbase[w] = acc;
+                acc += t;
+                most = t > most ? t : most;
+            }
+            s_wbase[16] = acc;
+            s_wbase[17] = most;
+        }
+        __syncthreads();
+        n_cand = s_wbase[16];
+        int pos = s_wbase[wv];
+        if (s_wbase[17] <= kWaveCand) {
+            // close the gaps between the waves' lists
+            uint32_t ck[kWaveCand / 64];
+            int ci[kWaveCand / 64];
+#pragma unroll
+            for (int u = 0; u < kWaveCand / 64; ++u) {
+                ck[u] = s_ck[wv * kWaveCand + u * 64 + lane];
+                ci[u] = s_ci[wv * kWaveCand + u * 64 + lane];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < kWaveCand / 64; ++u)
+                if (u * 64 + lane < wcount) {
+                    s_ck[pos + u * 64 + lane] = ck[u];
+                    s_ci[pos + u * 64 + lane] = ci[u];
+                }
+        } else if (n_cand <= SAMPLE_CAND) {
+            // candidates crowd in one wave's range: a second scan writes them
+            for (int b = c_lo; b < c_hi; b += 256) {
+                float v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int i = b + u * 64 + lane;
+                    v[u] = x[i < n ? i : n - 1];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int i = b + u * 64 + lane;
+                    const bool in = i < c_hi && sample_key(v[u]) >= L;
+                    const unsigned long long bal = __ballot(in);
+                    if (in) {
+                        const int at = pos + __popcll(bal & ((1ull << lane) - 1));
+                        s_ck[at] = sample_key(v[u] / T);
+                        s_ci[at] = i;
+                    }
+                    pos += __popcll(bal);
+                }
             }
         }
         __syncthreads();
+    }
+    if (n_cand <= kPairLen) {
+        // (c) survivors: the k first by (quotient, index), each candidate
+        // ranked against all
+        if (tid < 4) s_ck[n_cand + tid] = 0;
+        __syncthreads();
+        const uint32_t key = tid < n_cand ? s_ck[tid] : 0;
+        int rank = 0;
+        if (tid < n_cand)
+            for (int j = 0; j < n_cand; j += 4) {
+                const uint4 q = *(const uint4*)&s_ck[j];
+                rank += (q.x > key || (q.x == key && j < tid)) + (q.y > key || (q.y == key && j + 1 < tid)) +
+                        (q.z > key || (q.z == key && j + 2 < tid)) + (q.w > key || (q.w == key && j + 3 < tid));
+            }
+        const bool keep = tid < n_cand && rank < k;
+        const int o = block_excl_scan1024(keep, s_scan, &m);
+        if (keep) {
+            s_idx[o] = s_ci[tid];
+            s_val[o] = sample_unkey(key);
+        }
+    } else if (n_cand <= SAMPLE_CAND) {
         lds_select(s_ck, n_cand, k, s_bins, s_pick, &th, &need);
         // (c) survivors among the candidates (index order), one segment each
         const int seg = (n_cand + 1023) / 1024;
@@ -1524,20 +1648,33 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
         const float mx = block_max1024(tid < m ? s_val[tid] : -INFINITY, s_red);
         if (tid < m) s_p[tid] = sample_exp(s_val[tid] - mx);
         __syncthreads();
-        if (tid == 0) {
-            float sum = 0.0f;
-            for (int i = 0; i < m; ++i) sum += s_p[i];
-            s_sum = sum;
+        if (wv == 0) {
+            const float t = wave_run(m, [&](int i) { return s_p[i]; }, [](float) { return false; }, nullptr);
+            if (lane == 0) s_sum = t;
         }
         __syncthreads();
         const float sum = s_sum;
         if (sum > 0.0f) {
             if (tid < m) s_p[tid] = s_p[tid] / sum;
+            if (tid >= m && tid < m + 4 && tid < SAMPLE_MAX_K) s_p[tid] = -1.0f;
             int np2 = 1;
             while (np2 < m) np2 <<= 1;
             s_ord[tid] = tid;                       // np2 <= 1024 positions
             __syncthreads();
-            for (int k2 = 2; k2 <= np2; k2 <<= 1)
+            if (m <= kPairLen) {
+                // each survivor ranked against all; beyond, a sort is less work
+                if (tid < m) {
+                    const float p = s_p[tid];
+                    int rank = 0;
+                    for (int j = 0; j < m; j += 4) {
+                        const float4 q = *(const float4*)&s_p[j];
+                        rank += (q.x > p || (q.x == p && j < tid)) + (q.y > p || (q.y == p && j + 1 < tid)) +
+                                (q.z > p || (q.z == p && j + 2 < tid)) + (q.w > p || (q.w == p && j + 3 < tid));
+                    }
+                    s_ord[rank] = tid;
+                }
+                __syncthreads();
+            } else for (int k2 = 2; k2 <= np2; k2 <<= 1)
                 for (int j2 = k2 >> 1; j2 > 0; j2 >>= 1) {
                     const int i = tid, p = i ^ j2;
                     if (i < np2 && p > i) {
@@ -1551,14 +1688,11 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
                     }
                     __syncthreads();
                 }
-            if (tid == 0) {
-                float cum = 0.0f;
-                int cut = m;
-                for (int r = 0; r < m; ++r) {
-                    cum += s_p[s_ord[r]];
-                    if (cum >= c.top_p) { cut = r + 1; break; }
-                }
-                s_pick[0] = cut;
+            if (wv == 0) {
+                int r;
+                (void)wave_run(m, [&](int i) { return s_p[s_ord[i]]; },
+                               [&](float cum) { return cum >= c.top_p; }, &r);
+                if (lane == 0) s_pick[0] = r + 1 < m ? r + 1 : m;
             }
             __syncthreads();
             if (tid < m && tid >= s_pick[0]) s_val[s_ord[tid]] = -INFINITY;
@@ -1578,22 +1712,18 @@ __global__ __launch_bounds__(1024) void sample_kernel(SampleArgs a) {
     const float mx = block_max1024(tid < m ? s_val[tid] : -INFINITY, s_red);
     if (tid < m) s_p[tid] = sample_exp(s_val[tid] - mx);
     __syncthreads();
+    if (wv != 0) return;
+    const float sum = wave_run(m, [&](int i) { return s_p[i]; }, [](float) { return false; }, nullptr);
+    const float inv = 1.0f / sum;
+    unsigned long long r = *a.rng;
+    r ^= r << 13;
+    r ^= r >> 7;
+    r ^= r << 17;
+    const float u = (float)(uint32_t)(r >> 33) / 2147483648.0f;
+    int at;
+    (void)wave_run(m, [&](int i) { return s_p[i] * inv; }, [&](float cum) { return u < cum; }, &at);
     if (tid == 0) {
-        float sum = 0.0f;
-        for (int i = 0; i < m; ++i) sum += s_p[i];
-        const float inv = 1.0f / sum;
-        unsigned long long r = *a.rng;
-        r ^= r << 13;
-        r ^= r >> 7;
-        r ^= r << 17;
-        const float u = (float)(uint32_t)(r >> 33) / 2147483648.0f;
-        float cum = 0.0f;
-        uint32_t tok = (uint32_t)(n - 1);
-        for (int i = 0; i < m; ++i) {
-            const float p = s_p[i] * inv;
-            cum += p;
-            if (u < cum) { tok = (uint32_t)s_idx[i]; break; }
-        }
+        const uint32_t tok = at < m ? (uint32_t)s_idx[at] : (uint32_t)(n - 1);
         *a.rng = r;
         if (a.out_u32) *a.out_u32 = tok;
         if (a.record && a.hist && a.hist_len) { a.hist[len] = tok; *a.hist_len = len + 1; }

@@ -219,3 +219,25 @@ def test_generate_device_sampling_matches_host_sampling():
             host = []
             m.generate_streaming(prompt, 40, sc, lambda t: host.append(t) or True)
             assert dev == host, (seed, sc.top_k)
+
+
+@pytest.mark.parametrize("V", [1000, 1025, 4097, 33000, 100278])
+@pytest.mark.parametrize("T", [1e-6, 0.6, 1.0, 3.0, 3e38, float("inf")])
+@pytest.mark.parametrize("shape", ["spread", "crowded", "ties"])
+def test_device_sampler_candidates_without_division(V, T, shape):
+    # candidates are found on the logits and divided afterwards: quotients that
+    # fall together at large T, overflow at small T, have no order at T = inf;
+    # many candidates in one wave's range (its list holds 256) or in all
+    rng = np.random.default_rng(V)
+    lg = (rng.standard_normal(V) * 2).astype(np.float32)
+    if shape == "crowded":
+        lg[V // 3: V // 3 + 700] = 9 + rng.random(min(700, V - V // 3)).astype(np.float32)
+    elif shape == "ties":
+        lg = np.round(lg * 64) / np.float32(64)
+    if T > 100:
+        lg = np.abs(lg) + np.float32(0.5)     # the device ranks a quotient of +0 above -0, the host ties them
+    hist = [int(t) for t in rng.integers(0, V, 257)]
+    for k, p, n_hist, window in ((1, 1.0, 0, 64), (40, 0.95, 256, 256), (300, 0.9, 257, 257), (900, 0.99, 30, 64)):
+        s, keep = _cfg(temperature=T, top_k=k, top_p=p, repetition_penalty=1.1, repetition_window=window)
+        (th, sh), (td, sd) = _both(lg, hist[:n_hist], 1, s, 0x9E3779B97F4A7C15 + k)
+        assert (td, sd) == (th, sh), (k, p, n_hist)
