@@ -1085,14 +1085,20 @@ int gemm_rows_launch(const GemvArgs& a, bool needs_scratch, hipStream_t st) {
         if (!dig) p = pg_plan(a.fmt, a.M, a.N, a.K, true, false);
     }
     float* partial = nullptr;
-    if (p.splits > 1) {
-        const int rc = skinny_partial_for(a, (size_t)p.splits * a.N * a.M * sizeof(float), &partial);
+    // a captured call of this shape goes without the digits and may split more:
+    // the thread's scratch is left large enough for it
+    int held = p.splits;
+    if (p.kind == PG_INT8 && !a.partial)
+        held = std::max(held, pg_plan(a.fmt, a.M, a.N, a.K, true, false).splits);
+    if (held > 1) {
+        const int rc = skinny_partial_for(a, (size_t)held * a.N * a.M * sizeof(float), &partial);
         if (rc && needs_scratch) return rc;
         if (rc) {                             // none to be had: the call works without
             clear_error();
             p = pg_plan(a.fmt, a.M, a.N, a.K, false, dig != nullptr);
         }
     }
+    if (p.splits == 1) partial = nullptr;
     int sh = 0;
     while ((1 << sh) < a.cpb) ++sh;
     if (p.kind == PG_INT8 && p.tile == 6) pi_go<6>(a, p, dig, partial, st);

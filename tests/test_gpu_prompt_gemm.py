@@ -1,8 +1,12 @@
 """The prompt chunks' and ragged batches' GEMMs at the edges of their tiles, rings and K splits."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
 from tests.gpu_util import Dev, lib
+from tests.test_gpu_kernels import _hip_runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +109,67 @@ def test_int8_digits_special_rows(orc):
     tol = (2.0**-24 * np.max(np.abs(x[rest]).astype(np.float64), 1)[:, None] * np.sum(np.abs(w64), 1)[None, :]
            + 8 * 2.0**-24 * np.abs(ref))
     assert np.all(np.abs(got[rest] - ref) <= tol)
+
+
+# int8 shapes whose plan without the digits (a captured call has none) splits K
+# more than the plan with them: six times against five, twice against not at all
+@pytest.mark.parametrize("n,M,K", [(300, 2048, 4096), (700, 2048, 1024)])
+def test_int8_captured_after_a_call_of_the_same_shape(orc, n, M, K):
+    print(f"int8 prompt gemm captured n={n} M={M} K={K}", flush=True)
+    hip = _hip_runtime()
+    rng = np.random.default_rng(n)
+    w = (rng.standard_normal((M, K)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    q, s = orc.int8_quantize(w)
+    w64, x64 = orc.int8_dequantize(q, s).astype(np.float64), x.astype(np.float64)
+    res = {}
+
+    def worker():                           # a thread of its own: its scratch starts empty
+        st, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+        try:
+            dw, ds, dx, dy = Dev(q), Dev(s), Dev(x), Dev(np.full((n, M), np.nan, np.float32))
+            assert hip.hipStreamCreate(C.byref(st)) == 0
+            lib().atlas_set_thread_stream(st)
+
+            def call():
+                return lib().atlas_gemm_skinny_f32(2, dw.ptr, ds.ptr, 0, dx.ptr, dy.ptr, M, n, K)
+
+            assert call() == 0
+            lib().atlas_stream_sync()
+            res["eager"] = dy.get()
+            assert hip.hipStreamBeginCapture(st, 0) == 0
+            res["code"] = call()
+            assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0
+            if res["code"]:
+                return
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            res["replays"] = []
+            for _ in range(3):
+                lib().atlas_memset_zero(dy.ptr, n * M * 4)     # eager work between replays
+                lib().atlas_stream_sync()
+                assert hip.hipGraphLaunch(exe, st) == 0
+                assert hip.hipStreamSynchronize(st) == 0
+                res["replays"].append(dy.get())
+        except BaseException as e:          # reported on the main thread
+            res["exc"] = e
+        finally:
+            lib().atlas_clear_thread_stream()
+            if exe.value:
+                hip.hipGraphExecDestroy(exe)
+            if graph.value:
+                hip.hipGraphDestroy(graph)
+            if st.value:
+                hip.hipStreamSynchronize(st)
+                hip.hipStreamDestroy(st)
+
+    t = threading.Thread(target=worker)
+    t.start()
+    t.join()
+    if "exc" in res:
+        raise res["exc"]
+    assert res["code"] == 0, lib().atlas_last_error()
+    # two bf16 parts of x and f32 sums, as above
+    ref, tol = x64 @ w64.T, (2.0**-16 + K * 2.0**-24) * (np.abs(x64) @ np.abs(w64).T)
+    for got in [res["eager"]] + res["replays"]:
+        assert np.all(np.abs(got.astype(np.float64) - ref) <= tol)
+        assert np.array_equal(got, res["replays"][0]) or got is res["eager"]
