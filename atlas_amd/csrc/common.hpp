@@ -35,7 +35,6 @@ enum ScratchSlot {
     SCR_FUSED_PART,     // atlas_attention_fused_f32 split partials
     SCR_FUSED_CNT,      // ... its merge counters (kept at zero by the kernel)
     SCR_ATTN_CNT,       // atlas_decode_attention merge counters (kept at zero)
-    SCR_DIGITS,         // prompt-GEMM int8 digits of the activations
     SCR_SAMPLE,         // atlas_sample_device: logits copy and settings
     SCR_N
 };

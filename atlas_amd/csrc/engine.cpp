@@ -133,8 +133,6 @@ struct atlas_model {
     // the model's own, so captured steps never point at shared scratch
     float* gemm_part = nullptr;
     size_t gemm_part_bytes = 0;
-    void* gemm_digits = nullptr;     // int8 prompt chunks: the activations' digits
-    size_t gemm_digits_bytes = 0;
     // bf16 / int8 prompt chunks (17..1024 rows): hipBLASLt context (null: the tiled kernel)
     BlasRows* blas = nullptr;
     bool fused = false;
@@ -255,8 +253,6 @@ int skinny(atlas_model* m, const DevMat& w, const float* x, float* y, int n, int
     a.y_stride_m = 1;
     a.partial = m->gemm_part;
     a.partial_bytes = m->gemm_part_bytes;
-    a.digits = m->gemm_digits;
-    a.digits_bytes = m->gemm_digits_bytes;
     a.blas = m->blas;
     return skinny_launch(a, m->st);
 }
@@ -1568,10 +1564,6 @@ ATLAS_API atlas_model* atlas_model_create(const atlas_model_config* cfg) {
         }
         if (need && dalloc(m, (void**)&m->gemm_part, need)) return fail(m);
         m->gemm_part_bytes = need;
-        if (m->big_prefill && c.post_norm && fmt == WF_I8) {
-            m->gemm_digits_bytes = gemm_rows_digits_bytes(R, std::max(d, c.ffn_hidden));
-            if (dalloc(m, &m->gemm_digits, m->gemm_digits_bytes)) return fail(m);
-        }
         // bf16 and int8 prompt chunks through hipBLASLt (bf16 1.6x the tiled
         // kernel's rate at 127 rows of the 7B shapes) only when the
         // environment sets ATLAS_PROMPT_BLAS=1.  Off by default: one process

@@ -43,9 +43,6 @@ struct GemvArgs {
     long ldw;                // bytes between weight rows (multiple of 16); 0 = packed rows
     float* partial;          // skinny / prompt GEMM split-K partials (null: the thread's scratch)
     size_t partial_bytes;    // ... their size
-    void* digits;            // prompt GEMM, int8 weights: the activations' int8 digits (null with
-                             // partial null: the thread's scratch; null with partial: do without)
-    size_t digits_bytes;     // ... their size
     // skinny_launch, host side: non-null with EPI_STORE and the caller's
     // partial buffer, a split-K launch of the 2-8-row direct-load kernels or
     // of the prompt GEMMs (9+ rows) leaves its partials
@@ -87,7 +84,6 @@ bool gemm_rows_ok(const GemvArgs& a);
 bool gemm_rows_fit(const GemvArgs& a);
 int gemm_rows_launch(const GemvArgs& a, bool needs_scratch, hipStream_t st);
 size_t gemm_rows_partial_bytes(int fmt, int M, int N, int K);    // covers every smaller N
-size_t gemm_rows_digits_bytes(int N, int K);                     // GemvArgs.digits of int8 weights
 // The bf16 and int8 prompt GEMMs through hipBLASLt (blas.cpp): X's rows split
 // into bf16 hi and lo rows (bf16 weights) or three int8 digit rows (int8
 // weights), one library GEMM of the weights against all of them (the weights

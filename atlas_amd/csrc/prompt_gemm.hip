@@ -675,202 +675,6 @@ __global__ __launch_bounds__(512) void few_rows_gemm_kernel(GemvArgs a, float* _
     }
 }
 
-// ---- int8 weights, many rows -------------------------------------------------------
-// From ~130 rows the vector units bound the int8 kernel above: every weight is
-// made bf16 (and every activation split) between the MFMAs.  Here the
-// activations become integers instead, once: row n is s_n (d0 + d1 / 254 +
-// d2 / 254^2) with three int8 digits and s_n = max |x[n]| / 127, so within
-// 2^-24 of the row's largest element, and v_mfma_i32_16x16x64_i8 (twice the
-// bf16 rate; three products where bf16 takes two) sums q . d exactly.  Measured
-// (us, 1024 rows of the 7B shapes, digits included): 22016 x 4096 429 -> 256,
-// 12288 x 4096 263 -> 135, 4096 x 11008 212 -> 149; error against 64 bits
-// 5e-6 -> 4e-7.  192 weight rows fill 196 registers (three int32 sums per tile);
-// 256 would not fit.
-constexpr float kDigit = 254.0f;
-constexpr int kDigitsK = 131072;       // 127 * 127 * K stays within an int32 sum
-
-// one block per row: digits [3][N][K], row scales [N] (NaN for a row with one)
-__global__ __launch_bounds__(256) void prompt_digits_kernel(const float* __restrict__ x, long sn, int N, int K,
-                                                            int8_t* __restrict__ out, float* __restrict__ xs) {
-    __shared__ float red[4];
-    __shared__ int bad[4];
-    const int n = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const f32x4* row = reinterpret_cast<const f32x4*>(x + (long)n * sn);
-    constexpr int KEEP = 12;                     // pieces per thread kept in registers: K <= 12288
-    f32x4 v[KEEP];
-    float mx = 0.f;
-    bool nan = false;
-    const int np = K >> 2;
-#pragma unroll
-    for (int j = 0; j < KEEP; ++j) {
-        const int p = threadIdx.x + 256 * j;
-        v[j] = p < np ? row[p] : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    auto see = [&](const f32x4 t) {
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w))));
-        nan |= t.x != t.x || t.y != t.y || t.z != t.z || t.w != t.w;
-    };
-#pragma unroll
-    for (int j = 0; j < KEEP; ++j) see(v[j]);
-    for (int p = threadIdx.x + 256 * KEEP; p < np; p += 256) see(row[p]);
-    mx = wave_max(mx);
-    const bool any = __any(nan);
-    if (lane == 0) {
-        red[wave] = mx;
-        bad[wave] = any;
-    }
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const float s = mx > 0.f ? mx / 127.0f : 1.0f, inv = 1.0f / s;
-    if (threadIdx.x == 0) xs[n] = bad[0] | bad[1] | bad[2] | bad[3] ? __builtin_nanf("") : s;
-    const long plane = (long)N * K;
-    auto put = [&](int p, const f32x4 t) {
-        uint32_t d[3] = {0u, 0u, 0u};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            // |t / s - q0| <= 1/2 (1 + 2^-21); the remainder t - q0 s is exact
-            const float q = t[e] * inv;
-            const float q0 = rintf(q);
-            const float r1 = fmaf(-q0, s, t[e]) * inv * kDigit, q1 = rintf(r1);
-            const float q2 = rintf((r1 - q1) * kDigit);
-            d[0] |= ((uint32_t)(int)q0 & 0xFFu) << (8 * e);
-            d[1] |= ((uint32_t)(int)q1 & 0xFFu) << (8 * e);
-            d[2] |= ((uint32_t)(int)q2 & 0xFFu) << (8 * e);
-        }
-        uint32_t* o = reinterpret_cast<uint32_t*>(out + (long)n * K) + p;
-        o[0] = d[0];
-        *reinterpret_cast<uint32_t*>(reinterpret_cast<int8_t*>(o) + plane) = d[1];
-        *reinterpret_cast<uint32_t*>(reinterpret_cast<int8_t*>(o) + 2 * plane) = d[2];
-    };
-#pragma unroll
-    for (int j = 0; j < KEEP; ++j) {
-        const int p = threadIdx.x + 256 * j;
-        if (p < np) put(p, v[j]);
-    }
-    for (int p = threadIdx.x + 256 * KEEP; p < np; p += 256) put(p, row[p]);
-}
-
-// Eight waves (2 x 4), MF weight tiles x 2 activation tiles x 3 digits each: 32 MF
-// weight rows x 128 activation rows.  Units of 128 k (one line per row), two in
-// LDS: after the barrier of unit u, unit u + 1 loads while u is computed.
-template <int MF>
-struct PiShape {
-    static constexpr int WAVES = 8, BM = 32 * MF, BN = 128;
-    static constexpr int W_BYTES = BM * 128, X_BYTES = 3 * BN * 128, UNIT = W_BYTES + X_BYTES;
-    static constexpr int W_LD = W_BYTES / 1024 / WAVES, X_LD = X_BYTES / 1024 / WAVES;
-    static constexpr int BYTES = 2 * UNIT;
-};
-
-template <int MF>
-__global__ __launch_bounds__(512) void prompt_gemm_i8_kernel(GemvArgs a, const int8_t* __restrict__ xq,
-                                                              const float* __restrict__ xs,
-                                                              float* __restrict__ partial, int units_per_split,
-                                                              int m_tiles, int n_tiles) {
-    using S = PiShape<MF>;
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
-    extern __shared__ __align__(1024) uint8_t lds[];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = lane >> 4, li = lane & 15;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int M = a.M, N = a.N, K = a.K;
-    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int nt = idx % n_tiles, mt = (idx / n_tiles) * 8 + xcd;
-    if (mt >= m_tiles) return;
-    const int m0 = mt * S::BM, n0 = nt * S::BN;
-    const int u0 = blockIdx.y * units_per_split;
-    const int nunits = min(K / 128, u0 + units_per_split) - u0;
-
-    const long ldw = a.ldw > 0 ? a.ldw : (long)K;
-    const uint8_t* wbase = uniform_ptr(reinterpret_cast<const uint8_t*>(a.w) + (long)m0 * ldw + (long)u0 * 128);
-    const uint8_t* xbase = uniform_ptr(reinterpret_cast<const uint8_t*>(xq) + (long)n0 * K + (long)u0 * 128);
-    uint32_t woff[S::W_LD], xoff[S::X_LD];
-    const int lr = lane >> 3, lc = ((lane & 7) ^ lr) << 4;       // 8 rows per load, chunk c in slot c ^ row
-#pragma unroll
-    for (int j = 0; j < S::W_LD; ++j)
-        woff[j] = (uint32_t)((long)min((wave + 8 * j) * 8 + lr, M - 1 - m0) * ldw + lc);
-#pragma unroll
-    for (int j = 0; j < S::X_LD; ++j) {
-        const int inst = wave + 8 * j, p = inst >> 4, r = (inst & 15) * 8 + lr;
-        xoff[j] = (uint32_t)(((long)p * N + min(r, N - 1 - n0)) * K + lc);
-    }
-    const auto wsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wbase), 0, 0xFFFFFFFFu, 0x00020000);
-    const auto xsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(xbase), 0, 0xFFFFFFFFu, 0x00020000);
-    auto issue = [&](int u) {
-        uint8_t* st = lds + (u & 1) * S::UNIT;
-#pragma unroll
-        for (int j = 0; j < S::W_LD; ++j) load_lds<16>(wsrc, woff[j], u * 128, st + (wave + 8 * j) * 1024);
-#pragma unroll
-        for (int j = 0; j < S::X_LD; ++j)
-            load_lds<16>(xsrc, xoff[j], u * 128, st + S::W_BYTES + (wave + 8 * j) * 1024);
-    };
-
-    const int wofs = (wm * MF * 16 + li) * 128, xofs = S::W_BYTES + (wn * 32 + li) * 128;
-    i32x4 acc[3][2][MF];
-#pragma unroll
-    for (int p = 0; p < 3; ++p)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int i = 0; i < MF; ++i) acc[p][j][i] = i32x4{0, 0, 0, 0};
-    issue(0);
-    for (int u = 0; u < nunits; ++u) {
-        sync_stage<0>();
-        if (u + 1 < nunits) issue(u + 1);
-        const uint8_t* st = lds + (u & 1) * S::UNIT;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int c = ((4 * q + g) ^ (li & 7)) << 4;
-            i32x4 w[MF], xd[2][3];
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int p = 0; p < 3; ++p)
-                    xd[j][p] = *reinterpret_cast<const i32x4*>(st + xofs + (p * 128 + 16 * j) * 128 + c);
-#pragma unroll
-            for (int i = 0; i < MF; ++i) w[i] = *reinterpret_cast<const i32x4*>(st + wofs + i * 2048 + c);
-#pragma unroll
-            for (int i = 0; i < MF; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int p = 0; p < 3; ++p)
-                        acc[p][j][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xd[j][p], w[i], acc[p][j][i], 0, 0, 0);
-        }
-    }
-
-    // ---- epilogue: lane (g, li) holds D[4 g + v][li] of tile (j, i)
-    const int mb = m0 + wm * MF * 16 + li, nb = n0 + wn * 32 + 4 * g;
-    float rs[2][4];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) rs[j][v] = xs[min(nb + 16 * j + v, N - 1)];
-    const bool split_out = gridDim.y > 1;
-    float* y0 = split_out ? partial + (long)blockIdx.y * N * M + mb : a.y + (long)mb * a.y_stride_m;
-    const long sn = split_out ? M : a.y_stride_n, sm = split_out ? 16 : 16 * a.y_stride_m;
-#pragma unroll
-    for (int i = 0; i < MF; ++i) {
-        const float ws = a.scales[min(mb + 16 * i, M - 1)];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            f32x4 r;
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                r[v] = ((float)acc[0][j][i][v] +
-                        ((float)acc[1][j][i][v] + (float)acc[2][j][i][v] * (1.0f / kDigit)) * (1.0f / kDigit)) *
-                       rs[j][v] * ws;
-            if (!split_out && a.epi == EPI_SILU_MUL) {
-                pg_store_swiglu(a, r, mb + 16 * i, nb + 16 * j);
-            } else if (mb + 16 * i < M) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    if (nb + 16 * j + v < N) y0[(nb + 16 * j + v) * sn + i * sm] = r[v];
-            }
-        }
-    }
-}
-
 // ---- tile and K split ------------------------------------------------------------
 enum { PG_256x128, PG_192x128, PG_128x128, PG_256x64, PG_TILES };
 struct PgTile { int bm, bn; float step[3]; };      // us per k step of a block (bf16, int8, int4)
@@ -885,59 +689,48 @@ static constexpr float kFrUnit[3][3][2] = {{{0.50f, 0.95f}, {0.62f, 1.00f}, {0.9
                                            {{0.36f, 0.63f}, {0.45f, 0.79f}, {0.80f, 1.20f}},
                                            {{0.47f, 0.70f}, {0.59f, 0.94f}, {1.10f, 1.54f}}};
 constexpr int kFewRows = 64;
-// us per unit (128 k) of a block of the int8 kernel with 4 and 6 weight tiles per wave
-static constexpr float kPiUnit[2] = {1.40f, 1.80f};
-// steps: k steps per split of the tiled kernel; for the other two units of 128 k,
-// and tile is the weight tiles per wave
-enum { PG_TILED, PG_FEW, PG_INT8 };
-struct PgPlan { int kind, tile, splits, steps; };
+// few: the few-rows kernel, tile = weight tiles per wave (2, 4), steps = units of 128 k
+struct PgPlan { bool few; int tile, splits, steps; };
 
 static int pg_fmt(int fmt) { return fmt == WF_BF16 ? 0 : fmt == WF_I8 ? 1 : 2; }
 static int fr_nf(int N) { return N <= 16 ? 1 : N <= 32 ? 2 : 4; }
 
-// The kernel, tile and K split of least estimated time: rounds of one block per CU, each
+// The tile and K split of least estimated time: rounds of one block per CU, each
 // 4 us (first loads, stores) plus its k steps, and for a split the partials'
 // write and read at ~5 TB/s and the sum's launch.  Counted with N rounded up to
 // a tile, so that sizing at those N covers every N.  Measured against the
 // neighbours in this order (us, bf16): 127 rows gate/up 192 rows x 2 splits 64,
 // 256 x 2 68, 128 x 1 69; QKV 192 x 4 39, 256 x 4 42, 128 x 2 44; W_down
 // 128 x 8 37, 192 x 8 42; 24 rows gate/up 128 x 1 40, 64 x 1 48; W_down 64 x 4
-// 24, 128 x 8 25.  The int8 kernel pays for its digits (a read and a write of x)
-// from ~100 rows up: int8 gate/up at 127 rows 75 -> 51 us, 1024 rows 429 -> 256,
-// but W_o at 127 rows 20 -> 25; an estimate within 8% of the tiled kernel's
-// does not take it.
-static PgPlan pg_plan(int fmt, int M, int N, int K, bool split_ok, bool digits_ok) {
+// 24, 128 x 8 25.
+static PgPlan pg_plan(int fmt, int M, int N, int K, bool split_ok) {
     const int f = pg_fmt(fmt), cus = device_cu_count();
     PgPlan best{};
     float best_us = 0.f;
-    auto consider = [&](int kind, int tile, int bm, int bn, float step) {
-        const int total = kind == PG_TILED ? K / 32 : K / 128, unit = kind == PG_TILED ? 4 : 1;
+    auto consider = [&](bool few, int tile, int bm, int bn, float step) {
+        const int total = few ? K / 128 : K / 32, unit = few ? 1 : 4;
         const int nn = N <= kFewRows ? bn : (N + 63) / 64 * 64;
         const long tiles = (long)((M + bm - 1) / bm) * ((nn + bn - 1) / bn);
-        const float stream_us = kind == PG_FEW ? (float)M * gemv_row_bytes(fmt, K) / 5.5e6f : 0.f;
+        const float stream_us = few ? (float)M * gemv_row_bytes(fmt, K) / 5.5e6f : 0.f;
         for (int want = 1; want <= (split_ok ? 32 : 1); ++want) {
             const int steps = ((total + want - 1) / want + unit - 1) / unit * unit;
             const int splits = (total + steps - 1) / steps;
             if (splits != want) continue;
             const long rounds = (tiles * splits + cus - 1) / cus;
-            float us = kind == PG_FEW ? 4.f + std::max(rounds * steps * step, stream_us)
-                                      : rounds * (4.f + steps * step);
+            float us = few ? 4.f + std::max(rounds * steps * step, stream_us) : rounds * (4.f + steps * step);
             if (splits > 1) us += 3.f + (float)splits * nn * M * 8.f / 5e6f;
-            if (kind == PG_INT8) us = 1.08f * (us + 3.f + (float)nn * K * 7.f / 6.5e6f);
             if (best_us == 0.f || us < best_us) {
-                best = PgPlan{kind, tile, splits, steps};
+                best = PgPlan{few, tile, splits, steps};
                 best_us = us;
             }
         }
     };
     if (N <= 2 * kFewRows)
         for (int mf = 2; mf <= 4; mf += 2)
-            consider(PG_FEW, mf, 32 * mf, 16 * fr_nf(N), kFrUnit[f][fr_nf(N) >> 1][mf >> 2]);
+            consider(true, mf, 32 * mf, 16 * fr_nf(N), kFrUnit[f][fr_nf(N) >> 1][mf >> 2]);
     if (N > kFewRows)
         for (int t = 0; t < PG_TILES; ++t)
-            consider(PG_TILED, t, kPgTiles[t].bm, kPgTiles[t].bn, kPgTiles[t].step[f]);
-    if (N > kFewRows && digits_ok)
-        for (int mf = 4; mf <= 6; mf += 2) consider(PG_INT8, mf, 32 * mf, 128, kPiUnit[mf == 6]);
+            consider(false, t, kPgTiles[t].bm, kPgTiles[t].bn, kPgTiles[t].step[f]);
     return best;
 }
 
@@ -981,18 +774,18 @@ static void pg_launch(const GemvArgs& a, const PgPlan& p, float* partial, int sh
     const int nf = fr_nf(a.N);
     if constexpr (FMT != WF_BF16) {
         if (((uintptr_t)a.w | (uintptr_t)a.ldw) & 15) {
-            if (p.kind == PG_TILED) pg_go<FMT, 2, 4, 4, 2, 4>(a, p, partial, sh, st);
+            if (!p.few) pg_go<FMT, 2, 4, 4, 2, 4>(a, p, partial, sh, st);
             else if (nf == 1) fr_go<FMT, 2, 1, 4>(a, p, partial, sh, st);
             else if (nf == 2) fr_go<FMT, 2, 2, 4>(a, p, partial, sh, st);
             else fr_go<FMT, 2, 4, 4>(a, p, partial, sh, st);
             return;
         }
     }
-    if (p.kind == PG_FEW && p.tile == 2) {
+    if (p.few && p.tile == 2) {
         if (nf == 1) fr_go<FMT, 2, 1>(a, p, partial, sh, st);
         else if (nf == 2) fr_go<FMT, 2, 2>(a, p, partial, sh, st);
         else fr_go<FMT, 2, 4>(a, p, partial, sh, st);
-    } else if (p.kind == PG_FEW) {
+    } else if (p.few) {
         if (nf == 1) fr_go<FMT, 4, 1>(a, p, partial, sh, st);
         else if (nf == 2) fr_go<FMT, 4, 2>(a, p, partial, sh, st);
         else fr_go<FMT, 4, 4>(a, p, partial, sh, st);
@@ -1026,51 +819,11 @@ bool gemm_rows_fit(const GemvArgs& a) {
     return 256 * ldw < (1L << 32) && 128 * 4L * a.x_stride_n < (1L << 32) && a.K <= (1 << 23);
 }
 
-// whether the int8 kernel takes a (before asking for the digits' memory)
-static bool digits_fit(const GemvArgs& a) {
-    return a.fmt == WF_I8 && !a.f32x && (((uintptr_t)a.w | (uintptr_t)a.ldw) & 15) == 0 && a.K <= kDigitsK &&
-           3L * a.N * a.K < (1L << 31);
-}
-
-size_t gemm_rows_digits_bytes(int N, int K) { return (size_t)N * 4 + 16 + (size_t)3 * N * K; }
-
-// the caller's buffer, or the calling thread's scratch unless the stream is
-// being captured (a graph must not hold memory that no call before it needed)
-static uint8_t* digits_for(const GemvArgs& a, hipStream_t st) {
-    const size_t bytes = gemm_rows_digits_bytes(a.N, a.K);
-    if (a.digits) return bytes <= a.digits_bytes ? static_cast<uint8_t*>(a.digits) : nullptr;
-    if (a.partial) return nullptr;            // a model without a buffer of its own
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    void* p = nullptr;
-    if (thread_scratch(SCR_DIGITS, bytes, &p)) {
-        clear_error();
-        return nullptr;
-    }
-    return static_cast<uint8_t*>(p);
-}
-
-template <int MF>
-static void pi_go(const GemvArgs& a, const PgPlan& p, uint8_t* dig, float* partial, hipStream_t st) {
-    using S = PiShape<MF>;
-    float* xs = reinterpret_cast<float*>(dig);
-    int8_t* xq = reinterpret_cast<int8_t*>(dig) + ((size_t)a.N * 4 + 15) / 16 * 16;
-    const int mt = (a.M + S::BM - 1) / S::BM, nt = (a.N + S::BN - 1) / S::BN;
-    hipLaunchKernelGGL(prompt_digits_kernel, dim3(a.N), dim3(256), 0, st, a.x, a.x_stride_n, a.N, a.K, xq, xs);
-    hipLaunchKernelGGL(prompt_gemm_i8_kernel<MF>, dim3((mt + 7) / 8 * 8 * nt, p.splits), dim3(512), S::BYTES, st, a,
-                       xq, xs, partial, p.steps, mt, nt);
-}
-
 size_t gemm_rows_partial_bytes(int fmt, int M, int N, int K) {
     size_t need = 0;
     for (int n = 16; ; n = n < kFewRows ? 2 * n : n + 64) {
-        for (int dig = 0; dig < (fmt == WF_I8 ? 2 : 1); ++dig) {
-            const int sp = pg_plan(fmt, M, n, K, true, dig).splits;
-            if (sp > 1) need = std::max(need, (size_t)sp * std::min(n, N) * M * sizeof(float));
-        }
+        const int sp = pg_plan(fmt, M, n, K, true).splits;
+        if (sp > 1) need = std::max(need, (size_t)sp * std::min(n, N) * M * sizeof(float));
         if (n >= N) return need;
     }
 }
@@ -1078,32 +831,19 @@ size_t gemm_rows_partial_bytes(int fmt, int M, int N, int K) {
 int gemm_rows_launch(const GemvArgs& a, bool needs_scratch, hipStream_t st) {
     ATLAS_REQUIRE(gemm_rows_ok(a) && gemm_rows_fit(a), "gemm rows: unsupported shape (fmt %d, n %d, k %d)",
                   a.fmt, a.N, a.K);
-    PgPlan p = pg_plan(a.fmt, a.M, a.N, a.K, true, digits_fit(a));
-    uint8_t* dig = nullptr;
-    if (p.kind == PG_INT8) {
-        dig = digits_for(a, st);
-        if (!dig) p = pg_plan(a.fmt, a.M, a.N, a.K, true, false);
-    }
+    PgPlan p = pg_plan(a.fmt, a.M, a.N, a.K, true);
     float* partial = nullptr;
-    // a captured call of this shape goes without the digits and may split more:
-    // the thread's scratch is left large enough for it
-    int held = p.splits;
-    if (p.kind == PG_INT8 && !a.partial)
-        held = std::max(held, pg_plan(a.fmt, a.M, a.N, a.K, true, false).splits);
-    if (held > 1) {
-        const int rc = skinny_partial_for(a, (size_t)held * a.N * a.M * sizeof(float), &partial);
+    if (p.splits > 1) {
+        const int rc = skinny_partial_for(a, (size_t)p.splits * a.N * a.M * sizeof(float), &partial);
         if (rc && needs_scratch) return rc;
         if (rc) {                             // none to be had: the call works without
             clear_error();
-            p = pg_plan(a.fmt, a.M, a.N, a.K, false, dig != nullptr);
+            p = pg_plan(a.fmt, a.M, a.N, a.K, false);
         }
     }
-    if (p.splits == 1) partial = nullptr;
     int sh = 0;
     while ((1 << sh) < a.cpb) ++sh;
-    if (p.kind == PG_INT8 && p.tile == 6) pi_go<6>(a, p, dig, partial, st);
-    else if (p.kind == PG_INT8) pi_go<4>(a, p, dig, partial, st);
-    else if (a.fmt == WF_BF16) pg_launch<WF_BF16>(a, p, partial, sh, st);
+    if (a.fmt == WF_BF16) pg_launch<WF_BF16>(a, p, partial, sh, st);
     else if (a.fmt == WF_I8) pg_launch<WF_I8>(a, p, partial, sh, st);
     else pg_launch<WF_I4>(a, p, partial, sh, st);
     ATLAS_LAUNCH_CHECK("prompt_gemm");

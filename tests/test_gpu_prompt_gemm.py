@@ -65,16 +65,10 @@ def test_prompt_gemm(orc, fmt, n, M, K, block, off, epi):
     got = dy.get().astype(np.float64)
     x64 = x.astype(np.float64)
     ref, mag = x64 @ w64.T, np.abs(x64) @ np.abs(w64).T
-    if fmt == "int8":
-        # three digits, where they are taken: 2^-24 of the row's largest element per
-        # product, the sums exact, a few roundings to combine them
-        dig = 2.0**-24 * np.max(np.abs(x64), 1)[:, None] * np.sum(np.abs(w64), 1)[None, :] + 8 * 2.0**-24 * np.abs(ref)
     # x in two bf16 parts: the remainder of an 8-bit truncation rounded to 8 bits,
     # 2^-16 of each product; sums of K products in f32: K/2 roundings of 2^-24
     # (tree or chain, both within K 2^-24 of the magnitudes)
     tol = (2.0**-16 + K * 2.0**-24) * mag
-    if fmt == "int8":
-        tol = np.maximum(tol, dig)
     if fmt == "int4":
         # each step's 32 products run around the offset 24: 33 roundings of
         # sums of at most 32 s |x| per element
@@ -89,11 +83,52 @@ def test_prompt_gemm(orc, fmt, n, M, K, block, off, epi):
     assert np.all(np.abs(got - ref) <= tol), float(np.max(np.abs(got - ref) / tol))
 
 
-def test_int8_digits_special_rows(orc):
+def _sum_tol(x64, w64):
+    """|error| of Y = X W^T that x in two bf16 parts and f32 sums may show, per output, with S = |w x|_2:
+    each product's error is at most 2^-16 of it and zero in the mean, so 2e-11 of the outputs leave 7 * 2^-16 S
+    (Hoeffding); the same 7 S bounds the running sums, whose K / 16 additions (one per MFMA) and the few of the
+    K split and the scale each lose at most 2^-22 of them, the alignment of an MFMA's own products included."""
+    S = np.sqrt(np.square(x64) @ np.square(w64).T)
+    return 7 * (2.0**-16 + (x64.shape[1] / 16 + 8) * 2.0**-22) * S
+
+
+@pytest.mark.parametrize("n", [13, 60, 300])        # the few-rows and the tiled kernel
+@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+def test_rows_with_outliers_and_tiny_rows(orc, fmt, n):
+    # Every element keeps 16 bits of its own, whatever the rest of its row is: rows with one element 2^8 to 2^20
+    # times the others' size, whose weights there are stored as 0 in the first outputs; and rows so small that
+    # 127 / max |x| is no f32 number.
+    M, K = 6200, 1024
+    print(f"outliers and tiny rows {fmt} n={n}", flush=True)
+    rng = np.random.default_rng(11)
+    w = (rng.standard_normal((M, K)) * 0.02).astype(np.float32)
+    w[:M // 2, 100] = 0.0
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    tiny = np.arange(n) % 3 == 2
+    big = np.flatnonzero(~tiny)
+    x[big, 100] = 2.0 ** (8 + big % 13)
+    x[tiny] *= np.float32(1e-37)
+    data, scales, w64 = _stored(orc, w, fmt, 32)
+    dw, dx, dy = Dev(data), Dev(x), Dev(np.full((n, M), np.nan, np.float32))
+    ds = Dev(scales) if scales is not None else None
+    f = {"bf16": 1, "int8": 2, "int4": 3}[fmt]
+    assert lib().atlas_gemm_skinny_f32(f, dw.ptr, ds.ptr if ds else None, 32, dx.ptr, dy.ptr, M, n, K) == 0
+    got, x64 = dy.get().astype(np.float64), x.astype(np.float64)
+    err, tol = np.abs(got - x64 @ w64.T), _sum_tol(x64, w64)
+    assert np.all(err[~tiny] <= tol[~tiny]), float(np.max(err[~tiny] / tol[~tiny]))
+    # a tiny row's low parts are below 2^-126, where the matrix cores may take them for 0: 2^-7 of the element,
+    # all of one that is itself below; its f32 products with int8 or int4 weights are not
+    if fmt != "bf16":
+        tol = tol[tiny] + 7 * (2.0**-7 * np.sqrt(np.square(x64[tiny]) @ np.square(w64).T)
+                               + 2.0**-126 * np.sqrt(np.sum(np.square(w64), 1)))
+        assert np.all(err[tiny] <= tol), float(np.max(err[tiny] / tol))
+
+
+def test_int8_special_rows(orc):
     # rows with a NaN, an infinity, only zeros, one huge element; the others are
     # untouched by them
     n, M, K = 300, 6200, 512
-    print(f"int8 digits special rows n={n} M={M} K={K}", flush=True)
+    print(f"int8 special rows n={n} M={M} K={K}", flush=True)
     rng = np.random.default_rng(5)
     w = (rng.standard_normal((M, K)) * 0.02).astype(np.float32)
     x = rng.standard_normal((n, K)).astype(np.float32)
@@ -105,14 +140,11 @@ def test_int8_digits_special_rows(orc):
     got = dy.get().astype(np.float64)
     assert np.all(np.isnan(got[3])) and not np.any(np.isfinite(got[130])) and np.all(got[131] == 0)
     rest = [i for i in range(n) if i not in (3, 130)]
-    ref = x[rest].astype(np.float64) @ w64.T
-    tol = (2.0**-24 * np.max(np.abs(x[rest]).astype(np.float64), 1)[:, None] * np.sum(np.abs(w64), 1)[None, :]
-           + 8 * 2.0**-24 * np.abs(ref))
-    assert np.all(np.abs(got[rest] - ref) <= tol)
+    x64 = x[rest].astype(np.float64)
+    assert np.all(np.abs(got[rest] - x64 @ w64.T) <= _sum_tol(x64, w64))
 
 
-# int8 shapes whose plan without the digits (a captured call has none) splits K
-# more than the plan with them: six times against five, twice against not at all
+# shapes whose plan splits K six times and twice
 @pytest.mark.parametrize("n,M,K", [(300, 2048, 4096), (700, 2048, 1024)])
 def test_int8_captured_after_a_call_of_the_same_shape(orc, n, M, K):
     print(f"int8 prompt gemm captured n={n} M={M} K={K}", flush=True)
@@ -168,8 +200,6 @@ def test_int8_captured_after_a_call_of_the_same_shape(orc, n, M, K):
     if "exc" in res:
         raise res["exc"]
     assert res["code"] == 0, lib().atlas_last_error()
-    # two bf16 parts of x and f32 sums, as above
-    ref, tol = x64 @ w64.T, (2.0**-16 + K * 2.0**-24) * (np.abs(x64) @ np.abs(w64).T)
-    for got in [res["eager"]] + res["replays"]:
-        assert np.all(np.abs(got.astype(np.float64) - ref) <= tol)
-        assert np.array_equal(got, res["replays"][0]) or got is res["eager"]
+    assert np.all(np.abs(res["eager"].astype(np.float64) - x64 @ w64.T) <= _sum_tol(x64, w64))
+    for got in res["replays"]:
+        assert np.array_equal(got, res["eager"])
