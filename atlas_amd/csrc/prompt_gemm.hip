@@ -10,7 +10,7 @@
 //
 // MFMA operands (lane = 16 g + i): A = activations, lane (g, i) has k = 8g ..
 // 8g+7 of row i of a 16-row tile; B = weights, the same k of weight row i, as
-// stored (bf16) or made bf16 exactly (int8 q; int4 q + 24, see below); D: lane
+// stored (bf16) or made bf16 exactly (int8 q; int4 16 q, see below); D: lane
 // (g, i) has rows 4g .. 4g+3 of weight row i.
 //
 // What bounds it: with N in the hundreds the matrix cores (a bare loop of these
@@ -35,12 +35,13 @@
 //    their global addresses), so that fragment reads hit distinct banks.
 //  * The blocks of one weight tile run side by side on one XCD (its L2 then
 //    serves the weights to all but the first).
-//  * int4: word w's nibbles become bf16 by a shift and one mask-and-XOR per pair,
-//    q + 24 exactly; -24 * sum(x) comes from one more MFMA pair per activation
-//    tile as the start value of the step's products, which the block's scale
-//    multiplies (K % 32 == 0: a step is within one block).  (q + 136 saves one
-//    shift in eight, but its larger sums left 9.8e-6 of error where the exact
-//    conversions leave 8.6e-6.)
+//  * int4: the nibbles become 16 q exactly (each at the top of a byte, converted
+//    as int8 is), a step's products start from zero and are multiplied by the
+//    block's scale (K % 32 == 0: a step is within one block), the 1/16 by the
+//    epilogue.  (Masks alone give q + 24, whose -24 sum(x) has to be taken off
+//    again: nothing faster, 505 against 514 us at 22016 x 4096 and 1001 rows and
+//    310 against 288 at 12288 x 4096, but the larger sums cost every other element
+//    of a row with an outlier its low bits.)
 //
 // Measured (us; 7B shapes, against the one-launch-per-128-rows kernel before it):
 //   1024 rows          bf16          int8          int4
@@ -77,10 +78,12 @@ __device__ __forceinline__ void sync_stage() {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"i"(N) : "memory");
 }
 
+constexpr float kI4Unit = 16.0f;
+
 template <int FMT>
 using PgRaw = std::conditional_t<FMT == WF_BF16, u32x4, std::conditional_t<FMT == WF_I8, u32x2, uint32_t>>;
 
-// the bf16 parts of 8 activations (int4: in the order the nibble masks give).
+// the bf16 parts of 8 activations.
 // NS = 2: hi (truncation) and the rounded remainder; NS = 3: two truncations and
 // the rest, x exactly (8 + 8 + 8 bits).
 // The matrix cores round an f32 sum down, which shifts every result by about
@@ -89,17 +92,12 @@ using PgRaw = std::conditional_t<FMT == WF_BF16, u32x4, std::conditional_t<FMT =
 // prompt's logits against 1.5e-6).  So with three parts every other k step
 // multiplies -x and its sum is subtracted (flip, the sign bit): what one rounds
 // down the next rounds up.
-template <int FMT, int NS>
+template <int NS>
 __device__ __forceinline__ void pg_split(const f32x4 p, const f32x4 q, uint32_t flip, bf16x8 (&part)[NS]) {
     float e[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
     if constexpr (NS == 3)
 #pragma unroll
         for (int i = 0; i < 8; ++i) e[i] = __uint_as_float(__float_as_uint(e[i]) ^ flip);
-    if constexpr (FMT == WF_I4) {
-        const float o[8] = {p.y, q.y, p.x, q.x, p.w, q.w, p.z, q.z};
-#pragma unroll
-        for (int i = 0; i < 8; ++i) e[i] = o[i];
-    }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         u32x4 h;
@@ -113,10 +111,9 @@ __device__ __forceinline__ void pg_split(const f32x4 p, const f32x4 q, uint32_t 
     }
 }
 
-// 8 weights as a bf16 operand; nib: 0x00780078 in a vector register (one
-// mask-and-XOR per pair)
+// 8 weights as a bf16 operand (int4: times kI4Unit)
 template <int FMT>
-__device__ __forceinline__ bf16x8 pg_operand(const PgRaw<FMT> v, uint32_t nib) {
+__device__ __forceinline__ bf16x8 pg_operand(const PgRaw<FMT> v) {
     u32x4 b;
     if constexpr (FMT == WF_BF16) {
         b = v;
@@ -124,9 +121,11 @@ __device__ __forceinline__ bf16x8 pg_operand(const PgRaw<FMT> v, uint32_t nib) {
         b = u32x4{pack_f32_pair(s8_at(v.x, 0), s8_at(v.x, 1)), pack_f32_pair(s8_at(v.x, 2), s8_at(v.x, 3)),
                   pack_f32_pair(s8_at(v.y, 0), s8_at(v.y, 1)), pack_f32_pair(s8_at(v.y, 2), s8_at(v.y, 3))};
     } else {
-        // nibble q ^ 8 = q + 8 in the mantissa of 16: q + 24, exact in bf16
-        b = u32x4{((v << 3) & nib) ^ 0x41C041C0u, ((v >> 1) & nib) ^ 0x41C041C0u,
-                  ((v >> 5) & nib) ^ 0x41C041C0u, ((v >> 9) & nib) ^ 0x41C041C0u};
+        // element 2b in the high nibble of byte b: each nibble at the top of a
+        // byte is 16 q there
+        const uint32_t h = v & 0xF0F0F0F0u, l = (v << 4) & 0xF0F0F0F0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] = pack_f32_pair(s8_at(h, i), s8_at(l, i));
     }
     return __builtin_bit_cast(bf16x8, b);
 }
@@ -269,11 +268,9 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
     };
     // (three parts: odd steps with the sign turned)
     auto flip = [&](int s) { return (uint32_t)(s & 1) << 31; };
-    auto split_x = [&](int j, uint32_t f, bf16x8 (&part)[NS]) { pg_split<FMT, NS>(x0[j], x1[j], f, part); };
-    uint32_t nib = 0x00780078u;
-    if constexpr (FMT == WF_I4) asm("" : "+v"(nib));
+    auto split_x = [&](int j, uint32_t f, bf16x8 (&part)[NS]) { pg_split<NS>(x0[j], x1[j], f, part); };
     auto conv_w = [&](int i) {
-        if constexpr (FMT != WF_BF16) b[i] = pg_operand<FMT>(w[i], nib);
+        if constexpr (FMT != WF_BF16) b[i] = pg_operand<FMT>(w[i]);
     };
     auto w_op = [&](int i) -> bf16x8 {
         if constexpr (FMT == WF_BF16) return __builtin_bit_cast(bf16x8, w[i]);
@@ -285,16 +282,11 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
     for (int j = 0; j < NF; ++j)
 #pragma unroll
         for (int i = 0; i < MF; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const u32x4 neg24 = u32x4{0xC1C0C1C0u, 0xC1C0C1C0u, 0xC1C0C1C0u, 0xC1C0C1C0u};
 
     // activation tile j against every weight tile; last: each weight tile's
     // registers take the next step's tile as soon as it is done
     auto mfma_group = [&](const bf16x8 (&xp)[NS], int j, float sgn, const uint8_t* wst, int q, bool last) {
         if constexpr (FMT == WF_I4) {
-            const bf16x8 off = __builtin_bit_cast(bf16x8, neg24);
-            f32x4 d0 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s = 0; s < NS; ++s) d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[s], off, d0, 0, 0, 0);
             constexpr int H = MF / 2;
 #pragma unroll
             for (int h = 0; h < MF; h += H) {
@@ -303,7 +295,8 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
                 for (int s = 0; s < NS; ++s)
 #pragma unroll
                     for (int i = 0; i < H; ++i) {
-                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[s], w_op(h + i), s ? d[i] : d0, 0, 0, 0);
+                        d[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            xp[s], w_op(h + i), s ? d[i] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                         if (last && s + 1 == NS) conv_w(h + i);
                     }
 #pragma unroll
@@ -455,6 +448,11 @@ __global__ __launch_bounds__(64 * WM * WN) void prompt_gemm_kernel(GemvArgs a, f
 #pragma unroll
             for (int j = 0; j < NF; ++j) acc[j][i] *= rs;
         }
+    } else if constexpr (FMT == WF_I4) {
+#pragma unroll
+        for (int j = 0; j < NF; ++j)
+#pragma unroll
+            for (int i = 0; i < MF; ++i) acc[j][i] *= 1.0f / kI4Unit;
     }
     const bool split_out = gridDim.y > 1;
     if (!split_out && a.epi == EPI_SILU_MUL) {
@@ -577,9 +575,6 @@ __global__ __launch_bounds__(512) void few_rows_gemm_kernel(GemvArgs a, float* _
     for (int j = 0; j < NF; ++j)
 #pragma unroll
         for (int i = 0; i < MF; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8 off = __builtin_bit_cast(bf16x8, u32x4{0xC1C0C1C0u, 0xC1C0C1C0u, 0xC1C0C1C0u, 0xC1C0C1C0u});
-    uint32_t nib = 0x00780078u;
-    if constexpr (FMT == WF_I4) asm("" : "+v"(nib));
 
     auto compute = [&](int u) {
         const uint8_t* st = lds + (u % S::UR) * S::UNIT;
@@ -599,23 +594,15 @@ __global__ __launch_bounds__(512) void few_rows_gemm_kernel(GemvArgs a, float* _
         bf16x8 xp[NF][NS];
         const uint32_t flip = (uint32_t)(kg & 1) << 31;             // the step is KG u + kg
         const float sgn = (kg & 1) ? -1.0f : 1.0f;
-        f32x4 d0[FMT == WF_I4 ? NF : 1];
 #pragma unroll
-        for (int j = 0; j < NF; ++j) {
-            pg_split<FMT, NS>(x0[j], x1[j], flip, xp[j]);
-            if constexpr (FMT == WF_I4) {
-                d0[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int s = 0; s < NS; ++s) d0[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[j][s], off, d0[j], 0, 0, 0);
-            }
-        }
+        for (int j = 0; j < NF; ++j) pg_split<NS>(x0[j], x1[j], flip, xp[j]);
 #pragma unroll
         for (int i = 0; i < MF; ++i) {
-            const bf16x8 b = pg_operand<FMT>(w[i], nib);
+            const bf16x8 b = pg_operand<FMT>(w[i]);
             f32x4 d[NF];
 #pragma unroll
             for (int j = 0; j < NF; ++j)
-                d[j] = FMT == WF_I4 ? d0[FMT == WF_I4 ? j : 0] : NS == 3 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[j][i];
+                d[j] = FMT == WF_I4 || NS == 3 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[j][i];
 #pragma unroll
             for (int s = 0; s < NS; ++s)                       // (three parts: the small ones first)
 #pragma unroll
@@ -663,6 +650,7 @@ __global__ __launch_bounds__(512) void few_rows_gemm_kernel(GemvArgs a, float* _
         const int twm = t / (NF * MF), j = t / MF % NF, i = t % MF;
         const int m = m0 + (twm * MF + i) * 16 + li, nb = n0 + 16 * j + 4 * g;
         if constexpr (FMT == WF_I8) v *= a.scales[min(m, M - 1)];
+        if constexpr (FMT == WF_I4) v *= 1.0f / kI4Unit;
         if (!split_out && a.epi == EPI_SILU_MUL) {
             pg_store_swiglu(a, v, m, nb);
         } else if (m < M) {

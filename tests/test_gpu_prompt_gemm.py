@@ -69,11 +69,6 @@ def test_prompt_gemm(orc, fmt, n, M, K, block, off, epi):
     # 2^-16 of each product; sums of K products in f32: K/2 roundings of 2^-24
     # (tree or chain, both within K 2^-24 of the magnitudes)
     tol = (2.0**-16 + K * 2.0**-24) * mag
-    if fmt == "int4":
-        # each step's 32 products run around the offset 24: 33 roundings of
-        # sums of at most 32 s |x| per element
-        s_el = np.repeat(scales.astype(np.float64), block)[:M * K].reshape(M, K)
-        tol = tol + 33 * 2.0**-24 * (np.abs(x64) @ (32.0 * s_el).T)
     if epi == "swiglu":
         g, u, tg, tu = ref[:, 0::2], ref[:, 1::2], tol[:, 0::2], tol[:, 1::2]
         sg = 1.0 / (1.0 + np.exp(-g))
@@ -93,7 +88,7 @@ def _sum_tol(x64, w64):
 
 
 @pytest.mark.parametrize("n", [13, 60, 300])        # the few-rows and the tiled kernel
-@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+@pytest.mark.parametrize("fmt", ["bf16", "int8", "int4"])
 def test_rows_with_outliers_and_tiny_rows(orc, fmt, n):
     # Every element keeps 16 bits of its own, whatever the rest of its row is: rows with one element 2^8 to 2^20
     # times the others' size, whose weights there are stored as 0 in the first outputs; and rows so small that
