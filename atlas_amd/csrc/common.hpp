@@ -25,7 +25,8 @@ int device_cu_count();         // CUs of the current device (cached)
 // attention, split-K partials of the skinny GEMMs, argmax partials).  Each
 // slot grows stream-ordered on the thread's current stream (the old buffer is
 // freed after the work already queued there; a thread that switched streams
-// waits for the previous one first) and is kept until the thread exits.  Two
+// waits for the previous one first; one that a captured call used stays for
+// its graph) and is kept until the thread exits.  Two
 // threads never share a slot; calls of one thread on two streams at once do.
 // zero_new: a grown slot is cleared (fill kernel) before it is returned.
 enum ScratchSlot {

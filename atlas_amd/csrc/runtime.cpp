@@ -6,6 +6,8 @@
 // kernels/matmul.cu:580-595.
 #include <atomic>
 #include <mutex>
+#include <new>
+#include <vector>
 
 #include "common.hpp"
 #include "fused.hpp"
@@ -28,24 +30,32 @@ struct ScratchBuf {
     void* p = nullptr;
     size_t cap = 0;
     hipStream_t last = nullptr;   // stream of the most recent use
+    bool in_graph = false;        // a captured call points at p
 };
 struct ThreadScratch {
     ScratchBuf b[kScratchDevices][SCR_N];
+    // outgrown buffers that a graph's launches still write and read
+    std::vector<void*> held[kScratchDevices];
+    size_t held_bytes[kScratchDevices] = {};
     // a thread's slots go with it: each buffer is freed once the work queued
     // on the stream of its last use is done (hipFree waits for the device)
     ~ThreadScratch() {
         bool any = false;
         for (int d = 0; d < kScratchDevices; ++d)
             for (int i = 0; i < SCR_N; ++i) any = any || b[d][i].p;
+        for (const auto& h : held) any = any || !h.empty();
         if (!any) return;
         int cur = -1;
         if (hipGetDevice(&cur) != hipSuccess) return;
-        for (int d = 0; d < kScratchDevices; ++d)
+        for (int d = 0; d < kScratchDevices; ++d) {
             for (int i = 0; i < SCR_N; ++i)
                 if (b[d][i].p && hipSetDevice(d) == hipSuccess) {
                     (void)hipFree(b[d][i].p);
                     b[d][i].p = nullptr;
                 }
+            for (void* p : held[d])
+                if (hipSetDevice(d) == hipSuccess) (void)hipFree(p);
+        }
         (void)hipSetDevice(cur);
         (void)hipGetLastError();
     }
@@ -56,7 +66,7 @@ thread_local ThreadScratch t_scratch;
 size_t thread_scratch_bytes() {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) return 0;
-    size_t n = 0;
+    size_t n = t_scratch.held_bytes[dev];
     for (int i = 0; i < SCR_N; ++i) n += t_scratch.b[dev][i].cap;
     return n;
 }
@@ -69,12 +79,15 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
     ATLAS_REQUIRE(dev >= 0 && dev < kScratchDevices, "scratch: device %d", dev);
     ScratchBuf& s = t_scratch.b[dev][slot];
     hipStream_t st = stream();
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const hipError_t asked = hipStreamIsCapturing(st, &cs);
+    // (the null stream cannot be asked while another stream is captured)
+    if (asked != hipSuccess) (void)hipGetLastError();
     if (bytes > s.cap) {
         // Growing under a stream capture would record an allocation node
         // whose address is not backed until the graph runs (and the
         // synchronisation below would break the capture): refuse instead.
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        ATLAS_HIP(hipStreamIsCapturing(st, &cs));
+        ATLAS_HIP(asked);
         if (cs != hipStreamCaptureStatusNone) {
             set_error(ATLAS_EUNSUPPORTED,
                       "scratch: this call needs %zu bytes of library scratch on this thread and "
@@ -82,14 +95,22 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
                       "thread before the capture, or use a *_noalloc entry point", bytes);
             return ATLAS_EUNSUPPORTED;
         }
-        if (s.p) {
+        if (s.p && s.in_graph) {
+            // a graph keeps launching kernels on it: kept until the thread exits
+            try {
+                t_scratch.held[dev].push_back(s.p);
+            } catch (const std::bad_alloc&) {
+                set_error(ATLAS_ENOMEM, "scratch: no host memory");
+                return ATLAS_ENOMEM;
+            }
+            t_scratch.held_bytes[dev] += s.cap;
+        } else if (s.p) {
             // the old buffer may still be read by work queued on the stream
             // of its last use: free it after that work
             if (s.last != st) ATLAS_HIP(hipStreamSynchronize(s.last));
             ATLAS_HIP(hipFreeAsync(s.p, st));
-            s.p = nullptr;
-            s.cap = 0;
         }
+        s = ScratchBuf{};
         const size_t cap = (bytes + 65535) / 65536 * 65536;
         void* p = nullptr;
         if (dev_malloc_async(&p, cap, st) != hipSuccess || !p) {
@@ -108,7 +129,8 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
         s.p = p;
         s.cap = cap;
     }
-    s.last = st;
+    if (cs == hipStreamCaptureStatusNone) s.last = st;
+    else s.in_graph = true;
     *out = s.p;
     return ATLAS_OK;
 }

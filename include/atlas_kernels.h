@@ -33,7 +33,9 @@
  * thread exits.  A call that would grow it while its stream is being
  * captured into a graph returns / records ATLAS_EUNSUPPORTED instead: warm
  * up with one call of the same shape before the capture, or use
- * atlas_decode_attention_noalloc.
+ * atlas_decode_attention_noalloc.  A graph's launches use the scratch that
+ * its calls were captured with, which stays until the thread exits: order
+ * them with that thread's other calls.
  */
 #ifndef ATLAS_KERNELS_H
 #define ATLAS_KERNELS_H

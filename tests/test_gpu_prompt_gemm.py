@@ -198,3 +198,70 @@ def test_int8_captured_after_a_call_of_the_same_shape(orc, n, M, K):
     assert np.all(np.abs(res["eager"].astype(np.float64) - x64 @ w64.T) <= _sum_tol(x64, w64))
     for got in res["replays"]:
         assert np.array_equal(got, res["eager"])
+
+
+def _thread(fn):
+    """fn(res) on a thread of its own (its scratch starts empty); what it raises is raised here"""
+    res = {}
+
+    def worker():
+        try:
+            fn(res)
+        except BaseException as e:
+            res["exc"] = e
+        finally:
+            lib().atlas_clear_thread_stream()
+
+    t = threading.Thread(target=worker)
+    t.start()
+    t.join()
+    if "exc" in res:
+        raise res["exc"]
+    return res
+
+
+# A graph's K-split partials stay when a larger eager call outgrows them: the launches after it give the bits
+# of the ones before, and leave memory allocated since alone.
+def test_captured_scratch_outlives_growth(orc):
+    M, K, n, n2 = 2048, 8192, 64, 700
+    print(f"captured scratch outlives growth M={M} K={K} n={n} then {n2}", flush=True)
+    hip = _hip_runtime()
+    rng = np.random.default_rng(3)
+    w = orc.bf16_from_f32((rng.standard_normal((M, K)) * 0.02).astype(np.float32))
+    x = rng.standard_normal((n2, K)).astype(np.float32)
+
+    def run(res):
+        st, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+        dw, dx, dy, dz = Dev(w), Dev(x), Dev(np.zeros((n, M), np.float32)), Dev(np.zeros((n2, M), np.float32))
+        assert hip.hipStreamCreate(C.byref(st)) == 0
+        lib().atlas_set_thread_stream(st)
+        small = lambda: lib().atlas_gemm_skinny_f32(1, dw.ptr, None, 0, dx.ptr, dy.ptr, M, n, K)
+        try:
+            assert small() == 0
+            lib().atlas_stream_sync()
+            res["eager"], held = dy.get(), lib().atlas_thread_scratch_bytes()
+            assert held >= 2 * n * M * 4              # K is split
+            assert hip.hipStreamBeginCapture(st, 0) == 0
+            code = small()
+            assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0 and code == 0
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            assert lib().atlas_gemm_skinny_f32(1, dw.ptr, None, 0, dx.ptr, dz.ptr, M, n2, K) == 0
+            res["grown"] = lib().atlas_thread_scratch_bytes() - held
+            others = [Dev(np.full(held // 16, 5, np.float32)) for _ in range(8)]
+            for _ in range(3):
+                lib().atlas_memset_zero(dy.ptr, n * M * 4)
+                lib().atlas_stream_sync()
+                assert hip.hipGraphLaunch(exe, st) == 0
+                assert hip.hipStreamSynchronize(st) == 0
+                assert np.array_equal(dy.get(), res["eager"])
+            assert all(np.all(o.get() == 5) for o in others)
+        finally:
+            if exe.value:
+                hip.hipGraphExecDestroy(exe)
+            if graph.value:
+                hip.hipGraphDestroy(graph)
+            hip.hipStreamSynchronize(st)
+            hip.hipStreamDestroy(st)
+
+    # the larger call's buffer beside the graph's, which it does not replace
+    assert _thread(run)["grown"] >= 2 * n2 * M * 4
