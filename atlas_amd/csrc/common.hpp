@@ -26,8 +26,8 @@ int device_cu_count();         // CUs of the current device (cached)
 // slot grows stream-ordered on the thread's current stream (the old buffer is
 // freed after the work already queued there; a thread that switched streams
 // waits for the previous one first; one that a captured call used stays for
-// its graph) and is kept until the thread exits.  Two
-// threads never share a slot; calls of one thread on two streams at once do.
+// its graph) and is kept until the thread exits.  Two threads never share a
+// slot; a thread's call on another stream waits for the slot's last use.
 // zero_new: a grown slot is cleared (fill kernel) before it is returned.
 enum ScratchSlot {
     SCR_ATTN = 0,       // atlas_decode_attention split partials

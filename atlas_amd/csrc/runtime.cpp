@@ -4,6 +4,7 @@
 // (crates/atlas-tensor/src/lib.rs:151-161: cudaMalloc, cudaFree, cudaMemcpy,
 // cudaMallocAsync, cudaFreeAsync) and the device queries of
 // kernels/matmul.cu:580-595.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <new>
@@ -34,12 +35,15 @@ struct ScratchBuf {
 };
 struct ThreadScratch {
     ScratchBuf b[kScratchDevices][SCR_N];
+    hipEvent_t moved[kScratchDevices] = {};   // orders a slot's next stream behind its last
     // outgrown buffers that a graph's launches still write and read
     std::vector<void*> held[kScratchDevices];
     size_t held_bytes[kScratchDevices] = {};
     // a thread's slots go with it: each buffer is freed once the work queued
     // on the stream of its last use is done (hipFree waits for the device)
     ~ThreadScratch() {
+        for (hipEvent_t e : moved)
+            if (e) (void)hipEventDestroy(e);
         bool any = false;
         for (int d = 0; d < kScratchDevices; ++d)
             for (int i = 0; i < SCR_N; ++i) any = any || b[d][i].p;
@@ -61,6 +65,25 @@ struct ThreadScratch {
     }
 };
 thread_local ThreadScratch t_scratch;
+
+// `to` waits for what is queued on `from`, a stream its owner may have destroyed
+int order_streams(hipEvent_t& ev, hipStream_t from, hipStream_t to) {
+    if (!ev) ATLAS_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    if (hipEventRecord(ev, from) == hipSuccess) {
+        ATLAS_HIP(hipStreamWaitEvent(to, ev, 0));
+        return ATLAS_OK;
+    }
+    (void)hipGetLastError();
+    ATLAS_HIP(hipDeviceSynchronize());
+    return ATLAS_OK;
+}
+
+bool is_capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
 }  // namespace
 
 size_t thread_scratch_bytes() {
@@ -83,6 +106,19 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
     const hipError_t asked = hipStreamIsCapturing(st, &cs);
     // (the null stream cannot be asked while another stream is captured)
     if (asked != hipSuccess) (void)hipGetLastError();
+    // Work queued on the stream of the slot's last use may still read it: the
+    // next stream goes behind it.  (A captured call queues nothing.)  A stream
+    // being captured by now cannot be waited for: its buffer is left to it.
+    bool leave = s.in_graph;
+    if (s.p && s.last != st && cs == hipStreamCaptureStatusNone) {
+        if (is_capturing(s.last)) {
+            leave = true;
+            bytes = std::max(bytes, s.cap + 1);
+        } else {
+            const int rc = order_streams(t_scratch.moved[dev], s.last, st);
+            if (rc) return rc;
+        }
+    }
     if (bytes > s.cap) {
         // Growing under a stream capture would record an allocation node
         // whose address is not backed until the graph runs (and the
@@ -95,7 +131,7 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
                       "thread before the capture, or use a *_noalloc entry point", bytes);
             return ATLAS_EUNSUPPORTED;
         }
-        if (s.p && s.in_graph) {
+        if (s.p && leave) {
             // a graph keeps launching kernels on it: kept until the thread exits
             try {
                 t_scratch.held[dev].push_back(s.p);
@@ -105,10 +141,7 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
             }
             t_scratch.held_bytes[dev] += s.cap;
         } else if (s.p) {
-            // the old buffer may still be read by work queued on the stream
-            // of its last use: free it after that work
-            if (s.last != st) ATLAS_HIP(hipStreamSynchronize(s.last));
-            ATLAS_HIP(hipFreeAsync(s.p, st));
+            ATLAS_HIP(hipFreeAsync(s.p, st));        // after what is queued, as above
         }
         s = ScratchBuf{};
         const size_t cap = (bytes + 65535) / 65536 * 65536;

@@ -35,7 +35,9 @@
  * up with one call of the same shape before the capture, or use
  * atlas_decode_attention_noalloc.  A graph's launches use the scratch that
  * its calls were captured with, which stays until the thread exits: order
- * them with that thread's other calls.
+ * them with that thread's other calls.  A thread's call on another stream
+ * than its last waits for that stream's work where both use scratch; destroy
+ * no stream between the two.
  */
 #ifndef ATLAS_KERNELS_H
 #define ATLAS_KERNELS_H

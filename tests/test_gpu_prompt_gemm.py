@@ -265,3 +265,43 @@ def test_captured_scratch_outlives_growth(orc):
 
     # the larger call's buffer beside the graph's, which it does not replace
     assert _thread(run)["grown"] >= 2 * n2 * M * 4
+
+
+# One thread's calls on two streams share its split-K scratch: the second waits for the first.
+def test_scratch_of_two_streams(orc):
+    M, K, n = 4096, 11008, 127
+    print(f"scratch of two streams M={M} K={K} n={n}", flush=True)
+    hip = _hip_runtime()
+    rng = np.random.default_rng(4)
+    w = orc.bf16_from_f32((rng.standard_normal((M, K)) * 0.02).astype(np.float32))
+    xs = [rng.standard_normal((n, K)).astype(np.float32) for _ in range(4)]
+
+    def run(res):
+        streams = [C.c_void_p(), C.c_void_p()]
+        dw, dx = Dev(w), [Dev(x) for x in xs]
+        for st in streams:
+            assert hip.hipStreamCreate(C.byref(st)) == 0
+
+        def calls(pick, between):
+            out = [Dev(np.full((n, M), np.nan, np.float32)) for _ in xs]
+            lib().atlas_sync()
+            for i, (x, y) in enumerate(zip(dx, out)):
+                lib().atlas_set_thread_stream(streams[pick(i)])
+                assert lib().atlas_gemm_skinny_f32(1, dw.ptr, None, 0, x.ptr, y.ptr, M, n, K) == 0
+                between()
+            lib().atlas_sync()
+            return [y.get() for y in out]
+
+        try:
+            want = calls(lambda i: 0, lib().atlas_sync)
+            assert lib().atlas_thread_scratch_bytes() >= 2 * n * M * 4          # K is split
+            for _ in range(5):
+                got = calls(lambda i: i % 2, lambda: None)
+                assert all(np.array_equal(g, r) for g, r in zip(got, want))
+        finally:
+            lib().atlas_sync()
+            lib().atlas_clear_thread_stream()
+            for st in streams:
+                hip.hipStreamDestroy(st)
+
+    _thread(run)
