@@ -43,6 +43,7 @@ enum ScratchSlot {
 // ATLAS_EUNSUPPORTED (no allocation is recorded into the caller's graph).  A
 // thread's slots are freed when the thread exits.
 int thread_scratch(int slot, size_t bytes, void** out, bool zero_new = false);
+size_t thread_scratch_held(int slot);   // the slot's size on the current device
 size_t thread_scratch_bytes();   // bytes the calling thread holds on the current device
 
 // Check a HIP call; on failure record the error and return ATLAS_EHIP.

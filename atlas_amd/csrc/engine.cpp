@@ -1562,7 +1562,8 @@ ATLAS_API atlas_model* atlas_model_create(const atlas_model_config* cfg) {
                 need = std::max(need, gemm_rows_partial_bytes(
                                           fmt, sh[0], m->big_prefill && &sh != &shapes[4] ? R : nb, sh[1]));
         }
-        if (need && dalloc(m, (void**)&m->gemm_part, need)) return fail(m);
+        need = std::max(need, (size_t)256);      // never the calling thread's scratch
+        if (dalloc(m, (void**)&m->gemm_part, need)) return fail(m);
         m->gemm_part_bytes = need;
         // bf16 and int8 prompt chunks through hipBLASLt (bf16 1.6x the tiled
         // kernel's rate at 127 rows of the 7B shapes) only when the

@@ -78,11 +78,11 @@ int skinny_partial_for(const GemvArgs& a, size_t bytes, float** out);
 // Nine or more rows (2-8 of small matrices) of K % 128 == 0: the MFMA GEMMs of
 // prompt_gemm.hip (skinny_launch routes there) or, from 17 with a library context, the hipBLASLt prompt GEMM.
 // gemm_rows_ok: formats, alignment and strides they take; gemm_rows_fit: sizes
-// within their 32-bit offsets.  A call with needs_scratch false makes do
-// without a K split where the partials cannot be had.
+// within their 32-bit offsets.  Where the partials cannot be had a call makes do
+// with fewer K splits.
 bool gemm_rows_ok(const GemvArgs& a);
 bool gemm_rows_fit(const GemvArgs& a);
-int gemm_rows_launch(const GemvArgs& a, bool needs_scratch, hipStream_t st);
+int gemm_rows_launch(const GemvArgs& a, hipStream_t st);
 size_t gemm_rows_partial_bytes(int fmt, int M, int N, int K);    // covers every smaller N
 // The bf16 and int8 prompt GEMMs through hipBLASLt (blas.cpp): X's rows split
 // into bf16 hi and lo rows (bf16 weights) or three int8 digit rows (int8

@@ -676,7 +676,7 @@ static constexpr PgTile kPgTiles[PG_TILES] = {{256, 128, {0.83f, 1.02f, 1.30f}},
 static constexpr float kFrUnit[3][3][2] = {{{0.50f, 0.95f}, {0.62f, 1.00f}, {0.94f, 1.50f}},
                                            {{0.36f, 0.63f}, {0.45f, 0.79f}, {0.80f, 1.20f}},
                                            {{0.47f, 0.70f}, {0.59f, 0.94f}, {1.10f, 1.54f}}};
-constexpr int kFewRows = 64;
+constexpr int kFewRows = 64, kMaxSplits = 32;
 // few: the few-rows kernel, tile = weight tiles per wave (2, 4), steps = units of 128 k
 struct PgPlan { bool few; int tile, splits, steps; };
 
@@ -691,7 +691,7 @@ static int fr_nf(int N) { return N <= 16 ? 1 : N <= 32 ? 2 : 4; }
 // 256 x 2 68, 128 x 1 69; QKV 192 x 4 39, 256 x 4 42, 128 x 2 44; W_down
 // 128 x 8 37, 192 x 8 42; 24 rows gate/up 128 x 1 40, 64 x 1 48; W_down 64 x 4
 // 24, 128 x 8 25.
-static PgPlan pg_plan(int fmt, int M, int N, int K, bool split_ok) {
+static PgPlan pg_plan(int fmt, int M, int N, int K, int max_splits = kMaxSplits) {
     const int f = pg_fmt(fmt), cus = device_cu_count();
     PgPlan best{};
     float best_us = 0.f;
@@ -700,7 +700,7 @@ static PgPlan pg_plan(int fmt, int M, int N, int K, bool split_ok) {
         const int nn = N <= kFewRows ? bn : (N + 63) / 64 * 64;
         const long tiles = (long)((M + bm - 1) / bm) * ((nn + bn - 1) / bn);
         const float stream_us = few ? (float)M * gemv_row_bytes(fmt, K) / 5.5e6f : 0.f;
-        for (int want = 1; want <= (split_ok ? 32 : 1); ++want) {
+        for (int want = 1; want <= max_splits; ++want) {
             const int steps = ((total + want - 1) / want + unit - 1) / unit * unit;
             const int splits = (total + steps - 1) / steps;
             if (splits != want) continue;
@@ -807,26 +807,55 @@ bool gemm_rows_fit(const GemvArgs& a) {
     return 256 * ldw < (1L << 32) && 128 * 4L * a.x_stride_n < (1L << 32) && a.K <= (1 << 23);
 }
 
+// the row counts that pg_plan tells apart: 16, 32, 64 and every 64 from there
+static int pg_next_rows(int n) { return n < 16 ? 16 : n < kFewRows ? 2 * n : n + 64; }
+
 size_t gemm_rows_partial_bytes(int fmt, int M, int N, int K) {
     size_t need = 0;
-    for (int n = 16; ; n = n < kFewRows ? 2 * n : n + 64) {
-        const int sp = pg_plan(fmt, M, n, K, true).splits;
+    for (int n = 0; n < N;) {
+        n = pg_next_rows(n);
+        const int sp = pg_plan(fmt, M, n, K).splits;
         if (sp > 1) need = std::max(need, (size_t)sp * std::min(n, N) * M * sizeof(float));
-        if (n >= N) return need;
     }
+    return need;
 }
 
-int gemm_rows_launch(const GemvArgs& a, bool needs_scratch, hipStream_t st) {
+// What an eager call on the thread's scratch leaves there: enough for any
+// smaller N of the same weights (up to kHoldRows), so that such a call is
+// captured as it would run.  Fewer rows split K more: 4096 x 4096 not at all at
+// 1024 rows (76 us), eight times at 127 (21 us; 73 unsplit).  The plans are
+// looked at once per shape and thread (~1 us each).
+constexpr int kHoldRows = 1024;
+static size_t scratch_to_hold(const GemvArgs& a) {
+    struct Shape { int fmt, M, K, rows; size_t bytes; };
+    static thread_local Shape shapes[64] = {};
+    Shape& s = shapes[((unsigned)a.M * 31u + (unsigned)a.K * 7u + (unsigned)a.fmt) % 64u];
+    if (s.fmt != a.fmt || s.M != a.M || s.K != a.K)
+        s = Shape{a.fmt, a.M, a.K, 0, skinny_partial_bytes(a.M, 16, a.K)};
+    while (s.rows < std::min(a.N, kHoldRows)) {
+        s.rows = pg_next_rows(s.rows);
+        const int sp = pg_plan(a.fmt, a.M, s.rows, a.K).splits;
+        if (sp > 1) s.bytes = std::max(s.bytes, (size_t)sp * s.rows * a.M * sizeof(float));
+    }
+    return s.bytes;
+}
+
+int gemm_rows_launch(const GemvArgs& a, hipStream_t st) {
     ATLAS_REQUIRE(gemm_rows_ok(a) && gemm_rows_fit(a), "gemm rows: unsupported shape (fmt %d, n %d, k %d)",
                   a.fmt, a.N, a.K);
-    PgPlan p = pg_plan(a.fmt, a.M, a.N, a.K, true);
+    PgPlan p = pg_plan(a.fmt, a.M, a.N, a.K);
     float* partial = nullptr;
-    if (p.splits > 1) {
-        const int rc = skinny_partial_for(a, (size_t)p.splits * a.N * a.M * sizeof(float), &partial);
-        if (rc && needs_scratch) return rc;
-        if (rc) {                             // none to be had: the call works without
-            clear_error();
-            p = pg_plan(a.fmt, a.M, a.N, a.K, false);
+    const size_t split = (size_t)a.N * a.M * sizeof(float);
+    const size_t need = p.splits > 1 ? p.splits * split : 0, hold = a.partial ? need : scratch_to_hold(a);
+    if (std::max(need, hold) > 0 && skinny_partial_for(a, std::max(need, hold), &partial)) {
+        // Not to be had (no memory, or a capture on a thread that made no such
+        // call before it): what there is takes fewer splits, or none.
+        clear_error();
+        const size_t have = a.partial ? a.partial_bytes : thread_scratch_held(SCR_GEMM);
+        if (need > have) p = pg_plan(a.fmt, a.M, a.N, a.K, std::max(1, (int)(have / split)));
+        if (p.splits > 1) {
+            const int rc = skinny_partial_for(a, p.splits * split, &partial);
+            if (rc) return rc;
         }
     }
     int sh = 0;

@@ -94,6 +94,12 @@ size_t thread_scratch_bytes() {
     return n;
 }
 
+size_t thread_scratch_held(int slot) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) return 0;
+    return t_scratch.b[dev][slot].cap;
+}
+
 int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
     ATLAS_REQUIRE(out && slot >= 0 && slot < SCR_N, "scratch: bad slot %d", slot);
     *out = nullptr;

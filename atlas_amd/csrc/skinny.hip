@@ -1173,11 +1173,11 @@ static I4dPlan i4d_plan(int M, int K, int cus) {
 // Bytes of split-K partials an (M, N, K) launch needs; an N-row size
 // covers every smaller N.
 size_t skinny_partial_bytes(int M, int N, int K) {
-    int splits = skinny_splits(K, N);
-    if (N > 8) splits = std::max(splits, skinny_splits(K, 8));
-    else splits = std::max(splits, i4d_plan(M, K, device_cu_count()).splits);   // int4 rows
-    if (splits <= 1) return 0;
-    return (size_t)splits * N * M * sizeof(float);
+    const size_t row = (size_t)M * sizeof(float);
+    const int few = std::max(skinny_splits(K, 8), i4d_plan(M, K, device_cu_count()).splits);
+    size_t need = few > 1 ? few * std::min(N, 8) * row : 0;
+    if (N > 8 && skinny_splits(K, N) > 1) need = std::max(need, skinny_splits(K, N) * N * row);
+    return need;
 }
 
 template <int RM, int U>
@@ -1517,19 +1517,6 @@ static bool halves_pay(const GemvArgs& a) {
     return a.fmt == WF_BF16 && a.K > 4096;
 }
 
-// Whether this shape's rows have always needed split-K scratch, so that a call
-// that cannot have it is refused rather than run without a split.
-static bool rows_need_scratch(const GemvArgs& a) {
-    const int cus = device_cu_count();
-    if (a.N > 16) {
-        const int bx = (a.M + 127) / 128;
-        return bx < cus && !(a.fmt == WF_I4 && 5 * bx >= 3 * cus) && a.K >= 256;
-    }
-    if (a.N > 8 && !halves_pay(a)) return skinny_splits(a.K, a.N) > 1;
-    if (a.fmt != WF_I4 && a.K <= 4096) return false;
-    return i4d_plan(a.M, a.K, cus).splits > 1;
-}
-
 // Which rows take the few-rows and tiled GEMMs of prompt_gemm.hip (where
 // gemm_rows_ok): all from nine up; at the 7B shapes and 13 rows they take
 // 0.55-0.9x the time of the kernels below (bf16 W_down 41.5 -> 22.5 us, gate/up
@@ -1556,7 +1543,7 @@ int skinny_launch(const GemvArgs& a_in, hipStream_t st) {
     if (rows_ok && a.N > 16 && a.blas && !a.f32x && (a.fmt == WF_BF16 || (a.fmt == WF_I8 && a.K <= kDigitsMaxK)))
         return blas_rows_launch(a.blas, a, st);
     if (rows_ok && gemm_rows_fit(a) && (a.N > 16 || gemv_pitch_ok(a)))
-        return gemm_rows_launch(a, rows_need_scratch(a), st);
+        return gemm_rows_launch(a, st);
     ATLAS_REQUIRE(!a.f32x, "skinny: 24-bit activations need the prompt GEMMs' shapes (M %d K %d)", a.M, a.K);
     if (rows_ok && a.N > 16) {               // rows too long for their offsets: 16 at a time
         for (int n0 = 0; n0 < a.N; n0 += 16) {

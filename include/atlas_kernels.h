@@ -33,7 +33,11 @@
  * thread exits.  A call that would grow it while its stream is being
  * captured into a graph returns / records ATLAS_EUNSUPPORTED instead: warm
  * up with one call of the same shape before the capture, or use
- * atlas_decode_attention_noalloc.  A graph's launches use the scratch that
+ * atlas_decode_attention_noalloc.  (atlas_gemm_skinny_f32 with nine or more
+ * rows and k % 128 == 0 never needs it: short of scratch it splits k less,
+ * which is slower and sums in another order.  A call of n rows leaves enough
+ * for up to min(n, 1024) rows of the same weights, 34 to 158 MB after 1024 rows
+ * of a 7B matrix.)  A graph's launches use the scratch that
  * its calls were captured with, which stays until the thread exits: order
  * them with that thread's other calls.  A thread's call on another stream
  * than its last waits for that stream's work where both use scratch; destroy

@@ -305,3 +305,85 @@ def test_scratch_of_two_streams(orc):
                 hip.hipStreamDestroy(st)
 
     _thread(run)
+
+
+def _rand_weights(fmt, M, K, seed):
+    rng = np.random.default_rng(seed)
+    if fmt == "bf16":
+        w = (rng.standard_normal((M, K), np.float32) * np.float32(0.02)).view(np.uint32) >> 16
+        return w.astype(np.uint16), None
+    q = rng.integers(0, 256, M * K // (2 if fmt == "int4" else 1)).astype(np.uint8)
+    return q, rng.uniform(1e-4, 2e-4, M if fmt == "int8" else M * K // 32).astype(np.float32)
+
+
+def _eager_then_captured(fmt, M, K, rows, seed=9):
+    """On a thread of its own: eager calls of all but the last of `rows`, then one of the last recorded and
+    replayed three times.  (the last call's code, the replays, the data)"""
+    hip = _hip_runtime()
+    data, scales = _rand_weights(fmt, M, K, seed)
+    x = np.random.default_rng(seed + 1).standard_normal((max(rows), K), np.float32)
+    f = {"bf16": 1, "int8": 2, "int4": 3}[fmt]
+
+    def run(res):
+        st, graph, exe = C.c_void_p(), C.c_void_p(), C.c_void_p()
+        dw, dx, ds = Dev(data), Dev(x), Dev(scales) if scales is not None else None
+        dy, n = Dev(np.zeros((max(rows), M), np.float32)), rows[-1]
+        assert hip.hipStreamCreate(C.byref(st)) == 0
+        lib().atlas_set_thread_stream(st)
+        call = lambda r: lib().atlas_gemm_skinny_f32(f, dw.ptr, ds.ptr if ds else None, 32, dx.ptr, dy.ptr, M, r, K)
+        try:
+            for r in rows[:-1]:
+                assert call(r) == 0
+            lib().atlas_stream_sync()
+            assert hip.hipStreamBeginCapture(st, 0) == 0
+            res["code"] = call(n)
+            assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0
+            if res["code"]:
+                return
+            assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, C.c_size_t(0)) == 0
+            res["got"] = []
+            for _ in range(3):
+                lib().atlas_memset_zero(dy.ptr, n * M * 4)     # eager work between replays
+                lib().atlas_stream_sync()
+                assert hip.hipGraphLaunch(exe, st) == 0
+                assert hip.hipStreamSynchronize(st) == 0
+                res["got"].append(dy.get()[:n])
+            assert call(n) == 0
+            lib().atlas_stream_sync()
+            res["eager"] = dy.get()[:n]
+        finally:
+            if exe.value:
+                hip.hipGraphExecDestroy(exe)
+            if graph.value:
+                hip.hipGraphDestroy(graph)
+            hip.hipStreamSynchronize(st)
+            hip.hipStreamDestroy(st)
+
+    res = _thread(run)
+    return res["code"], res.get("got"), res.get("eager"), data, x[:rows[-1]]
+
+
+# fewer rows split K more, or take another kernel: 8 times against not at all, twice against not at all
+@pytest.mark.parametrize("fmt,M,K,rows", [("bf16", 4096, 4096, (1024, 127)), ("int8", 22016, 4096, (1024, 127)),
+                                          ("int4", 4096, 11008, (13, 6)), ("int4", 4096, 11008, (300, 6)),
+                                          ("bf16", 4096, 11008, (40, 16, 9))])
+def test_captured_after_a_larger_call(fmt, M, K, rows):
+    print(f"captured after a larger call {fmt} M={M} K={K} rows={rows}", flush=True)
+    code, got, eager, _, _ = _eager_then_captured(fmt, M, K, rows)
+    assert code == 0, lib().atlas_last_error()
+    assert all(np.array_equal(g, eager) for g in got)
+
+
+# with no scratch, or too little, K is split less
+@pytest.mark.parametrize("rows", [(64,), (13,), (128, 1000)])
+def test_captured_with_less_scratch(rows):
+    M, K = 2048, 8192
+    print(f"captured with less scratch M={M} K={K} rows={rows}", flush=True)
+    code, got, eager, data, x = _eager_then_captured("bf16", M, K, rows)
+    assert code == 0, lib().atlas_last_error()
+    w64 = (data.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    x64 = x.astype(np.float64)
+    ref, tol = x64 @ w64.T, _sum_tol(x64, w64)
+    assert np.all(np.abs(eager.astype(np.float64) - ref) <= tol)
+    for g in got:
+        assert np.array_equal(g, got[0]) and np.all(np.abs(g.astype(np.float64) - ref) <= tol)
