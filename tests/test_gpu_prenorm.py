@@ -94,3 +94,25 @@ def test_prompt_chunks_match_token_by_token(orc, fmt, tol, kw):
     got = m.generate_batch(prompts, 4)
     for p, g in zip(prompts, got):
         assert len(g) == 4 and g[0] == m.generate_with_sampling(p, 4, SamplingConfig.greedy())[0]
+
+
+# A 1B model's widths, in two layers so that every product of the first reaches the logits: chunks of 13, 30 and 60
+# rows take the few-rows kernel's 64- and 128-row blocks, 300 and 600 the four tiles (of 256 CUs: 256 x 64, 128 x 128,
+# 256 x 128; 128 x 128, 192 x 128, 256 x 128).  Running sums of K / 32 <= 256 steps walk to 2^-25 / sqrt(3) * 2
+# sqrt(256 / 2) = 4e-7 of their value, 16 of them to 1.6e-6, of the largest of the logits' differences and of the
+# logits alike; two and a half times that.  Two bf16 parts in place of three would leave 1.4e-5.
+@pytest.mark.parametrize("fmt", ["bf16", "int8"])
+def test_prompt_chunks_of_a_1b_layer(orc, fmt):
+    cfg = _cfg(d_model=2048, n_heads=16, n_kv_heads=4, ffn_hidden=8192, max_seq=640, sliding_window=0,
+               layer_sliding=[0, 0])
+    m = modelgen.engine_model(modelgen.make_weights(cfg, seed=31, fmt=fmt))
+    toks = [int(t) for t in np.random.default_rng(5).integers(0, cfg["vocab"], 601)]
+    for n in (13, 30, 60, 300, 600):
+        print(f"pre-norm 1B chunk {fmt} n={n}", flush=True)
+        got = []
+        for chunk in (1, 1024):
+            m.set_prefill_chunk(chunk)
+            m.reset()
+            m.prefill(toks[:n])
+            got.append(m.forward_one(toks[n]))
+        assert _rel(got[1], got[0]) <= 4e-6, n
