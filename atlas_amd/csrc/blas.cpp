@@ -2,8 +2,7 @@
 // through hipBLASLt.
 //
 // Y[n, m] = sum_k W[m, k] X[n, k] with W [M x K] (row pitch ldw) and X f32, as
-// the tiled kernel gemm_rows_kernel computes it (the prompt-chunk form of
-// Linear::forward, crates/atlas-model/src/lib.rs:487-499):
+// prompt_gemm.hip computes it (the prompt-chunk form of Linear::forward, crates/atlas-model/src/lib.rs:487-499):
 //  * bf16 weights: X's rows are split into bf16 hi and lo rows
 //    (split_rows_kernel, the tiled kernel's split), one library GEMM at f32
 //    accumulation multiplies the weights with all 2N rows, and

@@ -1565,8 +1565,7 @@ ATLAS_API atlas_model* atlas_model_create(const atlas_model_config* cfg) {
         need = std::max(need, (size_t)256);      // never the calling thread's scratch
         if (dalloc(m, (void**)&m->gemm_part, need)) return fail(m);
         m->gemm_part_bytes = need;
-        // bf16 and int8 prompt chunks through hipBLASLt (bf16 1.6x the tiled
-        // kernel's rate at 127 rows of the 7B shapes) only when the
+        // bf16 and int8 prompt chunks through hipBLASLt only when the
         // environment sets ATLAS_PROMPT_BLAS=1.  Off by default: one process
         // that had created and destroyed two library contexts (and run an
         // int4 model between) saw the library report that it could not

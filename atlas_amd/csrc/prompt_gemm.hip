@@ -43,17 +43,21 @@
 //    310 against 288 at 12288 x 4096, but the larger sums cost every other element
 //    of a row with an outlier its low bits.)
 //
-// Measured (us; 7B shapes, against the one-launch-per-128-rows kernel before it):
+// Measured (us; 7B shapes, the same weights call after call, against the
+// one-launch-per-128-rows kernel before it):
 //   1024 rows          bf16          int8          int4
-//   22016 x 4096       617 -> 341    620 -> 411    1164 -> 516    (+ SwiGLU)
-//   12288 x 4096       443 -> 192    455 -> 229     826 -> 301
-//   4096 x 4096        202 ->  76    213 ->  86     270 -> 103
-//   4096 x 11008       348 -> 175    362 -> 205     484 -> 252
+//   22016 x 4096       595 -> 335    613 -> 409    1158 -> 526    (+ SwiGLU)
+//   12288 x 4096       431 -> 191    450 -> 235     821 -> 309
+//   4096 x 4096        201 ->  75    214 ->  93     270 -> 113
+//   4096 x 11008       342 -> 175    357 -> 211     482 -> 263
 //   127 rows
-//   22016 x 4096        87 ->  64     84 ->  71     147 ->  90
-//   12288 x 4096        61 ->  39     60 ->  46     105 ->  56
-//   4096 x 4096         25 ->  21     27 ->  23      34 ->  27
-//   4096 x 11008        46 ->  37     49 ->  42      64 ->  50
+//   22016 x 4096        75 ->  56     77 ->  66     143 ->  88
+//   12288 x 4096        55 ->  37     57 ->  41     102 ->  52
+//   4096 x 4096         25 ->  22     27 ->  20      34 ->  24
+//   4096 x 11008        43 ->  36     45 ->  36      59 ->  43
+// Counters at 1024 rows (22016 x 4096; SIMD cycles): MFMAs 47% of them in bf16,
+// 36 in int8, 27 in int4; vector instructions (4 cycles each) 38, 55 and 63: two
+// MFMAs per product bound bf16, making the weights bf16 the other two.
 #include <algorithm>
 #include <type_traits>
 

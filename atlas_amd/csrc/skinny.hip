@@ -1518,10 +1518,10 @@ static bool halves_pay(const GemvArgs& a) {
 }
 
 // Which rows take the few-rows and tiled GEMMs of prompt_gemm.hip (where
-// gemm_rows_ok): all from nine up; at the 7B shapes and 13 rows they take
-// 0.55-0.9x the time of the kernels below (bf16 W_down 41.5 -> 22.5 us, gate/up
-// 47.9 -> 38.6, int8 29.4 -> 16.3 and 39.9 -> 24.1, int4 25.3 -> 15.6 and
-// 29.3 -> 26.5).  Of 2-8 rows those of small matrices, where the kernels below
+// gemm_rows_ok): all from nine up; at the 7B shapes and 13 rows, weights from
+// HBM, they take 0.5-0.9x the time of the kernels below (bf16 W_down 41.2 -> 23.9
+// us, gate/up 45.0 -> 40.3, int8 29.1 -> 15.1 and 39.6 -> 24.2, int4 25.3 -> 16.7;
+// int4 gate/up 28.1 -> 29.0, with exact weights in place of offset ones).  Of 2-8 rows those of small matrices, where the kernels below
 // leave CUs idle (4 rows, us: bf16 2048 x 8192 14.6 -> 10.2, 8192 x 2048
 // 11.3 -> 9.3, 640 x 640 7.5 -> 4.1; int8 9.2 -> 9.1, 9.5 -> 8.7, 6.6 -> 4.5);
 // from there up their streaming is the faster one (bf16 12288 x 4096 19.7

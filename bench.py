@@ -297,7 +297,7 @@ def decode_bench(model_mod, fmt: int, prompt, steps: int, warmup: int, seed: int
     # the prompt: token by token (the reference's loop), then through the
     # multi-row prefill step; the second leaves the state the decode continues
     pre = {}
-    # 128-row chunks take hipBLASLt (bf16, int8) or the tiled MFMA GEMM (int4)
+    # 128-row chunks take the few-rows and tiled MFMA GEMMs
     for chunk in (1, 16, 128):
         m.reset()
         m.set_prefill_chunk(chunk)
