@@ -23,11 +23,10 @@ int device_cu_count();         // CUs of the current device (cached)
 // Device scratch owned by the calling thread on the current device, for entry
 // points that are not handed a workspace (split partials of the reference-ABI
 // attention, split-K partials of the skinny GEMMs, argmax partials).  Each
-// slot grows stream-ordered on the thread's current stream (the old buffer is
-// freed after the work already queued there; a thread that switched streams
-// waits for the previous one first; one that a captured call used stays for
-// its graph) and is kept until the thread exits.  Two threads never share a
-// slot; a thread's call on another stream waits for the slot's last use.
+// slot has a buffer per stream that the thread calls on.  It grows
+// stream-ordered (the old one is freed after the work already queued on its
+// stream; one that a captured call used stays for its graph) and is kept until
+// the thread exits.  Two threads never share a buffer.
 // zero_new: a grown slot is cleared (fill kernel) before it is returned.
 enum ScratchSlot {
     SCR_ATTN = 0,       // atlas_decode_attention split partials
@@ -43,7 +42,7 @@ enum ScratchSlot {
 // ATLAS_EUNSUPPORTED (no allocation is recorded into the caller's graph).  A
 // thread's slots are freed when the thread exits.
 int thread_scratch(int slot, size_t bytes, void** out, bool zero_new = false);
-size_t thread_scratch_held(int slot);   // the slot's size on the current device
+size_t thread_scratch_held(int slot);   // what a call on the current stream has of it
 size_t thread_scratch_bytes();   // bytes the calling thread holds on the current device
 
 // Check a HIP call; on failure record the error and return ATLAS_EHIP.

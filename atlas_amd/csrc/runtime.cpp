@@ -4,8 +4,8 @@
 // (crates/atlas-tensor/src/lib.rs:151-161: cudaMalloc, cudaFree, cudaMemcpy,
 // cudaMallocAsync, cudaFreeAsync) and the device queries of
 // kernels/matmul.cu:580-595.
-#include <algorithm>
 #include <atomic>
+#include <cstdint>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -27,77 +27,78 @@ hipStream_t stream() { return t_has_stream ? t_stream : g_stream.load(std::memor
 
 namespace {
 constexpr int kScratchDevices = 16;
+// A slot has a buffer per stream that its thread calls on, so that calls queued
+// on two streams do not meet in it; beyond this many the one used longest ago
+// changes hands after a device synchronisation.  (The other streams' handles are
+// only compared: their owners may have destroyed them, and HIP crashes on one.)
+constexpr int kScratchStreams = 4;
 struct ScratchBuf {
     void* p = nullptr;
     size_t cap = 0;
-    hipStream_t last = nullptr;   // stream of the most recent use
+    hipStream_t owner = nullptr;
     bool in_graph = false;        // a captured call points at p
+    unsigned long used = 0;       // ThreadScratch::clock of the most recent use
 };
 struct ThreadScratch {
-    ScratchBuf b[kScratchDevices][SCR_N];
-    hipEvent_t moved[kScratchDevices] = {};   // orders a slot's next stream behind its last
+    ScratchBuf b[kScratchDevices][SCR_N][kScratchStreams];
+    unsigned long clock = 0;
     // outgrown buffers that a graph's launches still write and read
     std::vector<void*> held[kScratchDevices];
     size_t held_bytes[kScratchDevices] = {};
-    // a thread's slots go with it: each buffer is freed once the work queued
-    // on the stream of its last use is done (hipFree waits for the device)
+    // a thread's slots go with it (hipFree waits for the device)
     ~ThreadScratch() {
-        for (hipEvent_t e : moved)
-            if (e) (void)hipEventDestroy(e);
-        bool any = false;
-        for (int d = 0; d < kScratchDevices; ++d)
-            for (int i = 0; i < SCR_N; ++i) any = any || b[d][i].p;
-        for (const auto& h : held) any = any || !h.empty();
-        if (!any) return;
         int cur = -1;
-        if (hipGetDevice(&cur) != hipSuccess) return;
         for (int d = 0; d < kScratchDevices; ++d) {
-            for (int i = 0; i < SCR_N; ++i)
-                if (b[d][i].p && hipSetDevice(d) == hipSuccess) {
-                    (void)hipFree(b[d][i].p);
-                    b[d][i].p = nullptr;
-                }
-            for (void* p : held[d])
+            auto drop = [&](void* p) {
+                if (!p || (cur < 0 && hipGetDevice(&cur) != hipSuccess)) return;
                 if (hipSetDevice(d) == hipSuccess) (void)hipFree(p);
+            };
+            for (auto& slot : b[d])
+                for (ScratchBuf& s : slot) drop(s.p);
+            for (void* p : held[d]) drop(p);
         }
+        if (cur < 0) return;
         (void)hipSetDevice(cur);
         (void)hipGetLastError();
     }
 };
 thread_local ThreadScratch t_scratch;
 
-// `to` waits for what is queued on `from`, a stream its owner may have destroyed
-int order_streams(hipEvent_t& ev, hipStream_t from, hipStream_t to) {
-    if (!ev) ATLAS_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    if (hipEventRecord(ev, from) == hipSuccess) {
-        ATLAS_HIP(hipStreamWaitEvent(to, ev, 0));
-        return ATLAS_OK;
-    }
-    (void)hipGetLastError();
-    ATLAS_HIP(hipDeviceSynchronize());
-    return ATLAS_OK;
+int scratch_device() {
+    int dev = 0;
+    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kScratchDevices ? dev : -1;
 }
 
-bool is_capturing(hipStream_t st) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return false;
+// What a call on st uses of a slot: a captured one the stream's own buffer or,
+// where that is smaller than `bytes`, the largest; others their own (null: none yet).
+ScratchBuf* scratch_find(ScratchBuf (&slot)[kScratchStreams], hipStream_t st, bool captured, size_t bytes) {
+    ScratchBuf *own = nullptr, *big = nullptr;
+    for (ScratchBuf& s : slot) {
+        if (!s.p) continue;
+        if (s.owner == st) own = &s;
+        if (!big || s.cap > big->cap) big = &s;
+    }
+    return captured && (!own || own->cap < bytes) ? big : own;
 }
 }  // namespace
 
 size_t thread_scratch_bytes() {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) return 0;
+    const int dev = scratch_device();
+    if (dev < 0) return 0;
     size_t n = t_scratch.held_bytes[dev];
-    for (int i = 0; i < SCR_N; ++i) n += t_scratch.b[dev][i].cap;
+    for (const auto& slot : t_scratch.b[dev])
+        for (const ScratchBuf& s : slot) n += s.cap;
     return n;
 }
 
 size_t thread_scratch_held(int slot) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) return 0;
-    return t_scratch.b[dev][slot].cap;
+    const int dev = scratch_device();
+    if (dev < 0) return 0;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream(), &cs) != hipSuccess) (void)hipGetLastError();
+    const bool captured = cs != hipStreamCaptureStatusNone;
+    const ScratchBuf* s = scratch_find(t_scratch.b[dev][slot], stream(), captured, SIZE_MAX);
+    return s ? s->cap : 0;
 }
 
 int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
@@ -106,50 +107,45 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
     int dev = 0;
     ATLAS_HIP(hipGetDevice(&dev));
     ATLAS_REQUIRE(dev >= 0 && dev < kScratchDevices, "scratch: device %d", dev);
-    ScratchBuf& s = t_scratch.b[dev][slot];
+    auto& bufs = t_scratch.b[dev][slot];
     hipStream_t st = stream();
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     const hipError_t asked = hipStreamIsCapturing(st, &cs);
     // (the null stream cannot be asked while another stream is captured)
     if (asked != hipSuccess) (void)hipGetLastError();
-    // Work queued on the stream of the slot's last use may still read it: the
-    // next stream goes behind it.  (A captured call queues nothing.)  A stream
-    // being captured by now cannot be waited for: its buffer is left to it.
-    bool leave = s.in_graph;
-    if (s.p && s.last != st && cs == hipStreamCaptureStatusNone) {
-        if (is_capturing(s.last)) {
-            leave = true;
-            bytes = std::max(bytes, s.cap + 1);
-        } else {
-            const int rc = order_streams(t_scratch.moved[dev], s.last, st);
-            if (rc) return rc;
-        }
-    }
-    if (bytes > s.cap) {
+    const bool captured = cs != hipStreamCaptureStatusNone;
+    ScratchBuf* s = scratch_find(bufs, st, captured, bytes);
+    if (captured && (!s || s->cap < bytes)) {
         // Growing under a stream capture would record an allocation node
-        // whose address is not backed until the graph runs (and the
-        // synchronisation below would break the capture): refuse instead.
+        // whose address is not backed until the graph runs: refuse instead.
+        set_error(ATLAS_EUNSUPPORTED,
+                  "scratch: this call needs %zu bytes of library scratch on this thread and "
+                  "the stream is being captured; make one call of the same shape on this "
+                  "thread before the capture, or use a *_noalloc entry point", bytes);
+        return ATLAS_EUNSUPPORTED;
+    }
+    if (!s) {                                // the stream's first call
+        s = &bufs[0];
+        for (ScratchBuf& t : bufs)           // unused, else without a graph, else used longest ago
+            if (!t.p != !s->p ? !t.p : t.in_graph != s->in_graph ? s->in_graph : t.used < s->used) s = &t;
+        if (s->p) ATLAS_HIP(hipDeviceSynchronize());
+        s->owner = st;
+    }
+    if (bytes > s->cap) {
         ATLAS_HIP(asked);
-        if (cs != hipStreamCaptureStatusNone) {
-            set_error(ATLAS_EUNSUPPORTED,
-                      "scratch: this call needs %zu bytes of library scratch on this thread and "
-                      "the stream is being captured; make one call of the same shape on this "
-                      "thread before the capture, or use a *_noalloc entry point", bytes);
-            return ATLAS_EUNSUPPORTED;
-        }
-        if (s.p && leave) {
+        if (s->p && s->in_graph) {
             // a graph keeps launching kernels on it: kept until the thread exits
             try {
-                t_scratch.held[dev].push_back(s.p);
+                t_scratch.held[dev].push_back(s->p);
             } catch (const std::bad_alloc&) {
                 set_error(ATLAS_ENOMEM, "scratch: no host memory");
                 return ATLAS_ENOMEM;
             }
-            t_scratch.held_bytes[dev] += s.cap;
-        } else if (s.p) {
-            ATLAS_HIP(hipFreeAsync(s.p, st));        // after what is queued, as above
+            t_scratch.held_bytes[dev] += s->cap;
+        } else if (s->p) {
+            ATLAS_HIP(hipFreeAsync(s->p, st));       // after the work queued on its stream
         }
-        s = ScratchBuf{};
+        *s = ScratchBuf{};
         const size_t cap = (bytes + 65535) / 65536 * 65536;
         void* p = nullptr;
         if (dev_malloc_async(&p, cap, st) != hipSuccess || !p) {
@@ -165,12 +161,13 @@ int thread_scratch(int slot, size_t bytes, void** out, bool zero_new) {
                 return rc;
             }
         }
-        s.p = p;
-        s.cap = cap;
+        s->p = p;
+        s->cap = cap;
+        s->owner = st;
     }
-    if (cs == hipStreamCaptureStatusNone) s.last = st;
-    else s.in_graph = true;
-    *out = s.p;
+    s->in_graph = s->in_graph || captured;
+    s->used = ++t_scratch.clock;
+    *out = s->p;
     return ATLAS_OK;
 }
 

@@ -39,9 +39,9 @@
  * for up to min(n, 1024) rows of the same weights, 34 to 158 MB after 1024 rows
  * of a 7B matrix.)  A graph's launches use the scratch that
  * its calls were captured with, which stays until the thread exits: order
- * them with that thread's other calls.  A thread's call on another stream
- * than its last waits for that stream's work where both use scratch; destroy
- * no stream between the two.
+ * them with that thread's other calls.  A thread that calls on several
+ * streams has scratch for each of up to four; a fifth takes over the one used
+ * longest ago after a device synchronisation.
  */
 #ifndef ATLAS_KERNELS_H
 #define ATLAS_KERNELS_H

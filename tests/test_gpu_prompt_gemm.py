@@ -267,7 +267,7 @@ def test_captured_scratch_outlives_growth(orc):
     assert _thread(run)["grown"] >= 2 * n2 * M * 4
 
 
-# One thread's calls on two streams share its split-K scratch: the second waits for the first.
+# One thread's calls on two streams at once do not meet in its split-K scratch.
 def test_scratch_of_two_streams(orc):
     M, K, n = 4096, 11008, 127
     print(f"scratch of two streams M={M} K={K} n={n}", flush=True)
@@ -387,3 +387,56 @@ def test_captured_with_less_scratch(rows):
     assert np.all(np.abs(eager.astype(np.float64) - ref) <= tol)
     for g in got:
         assert np.array_equal(g, got[0]) and np.all(np.abs(g.astype(np.float64) - ref) <= tol)
+
+
+def test_no_memory_for_the_partials():
+    M, K, n = 2048, 8192, 64
+    print(f"no memory for the partials M={M} K={K} n={n}", flush=True)
+    data, _ = _rand_weights("bf16", M, K, 21)
+    x = np.random.default_rng(22).standard_normal((n, K), np.float32)
+
+    def run(res):
+        dw, dx, dy = Dev(data), Dev(x), Dev(np.full((n, M), np.nan, np.float32))
+        try:
+            lib().atlas_debug_fail_allocations(0, 2)
+            res["code"] = lib().atlas_gemm_skinny_f32(1, dw.ptr, None, 0, dx.ptr, dy.ptr, M, n, K)
+        finally:
+            lib().atlas_debug_fail_allocations(0, 0)
+        res["error"], res["bytes"] = lib().atlas_last_error_code(), lib().atlas_thread_scratch_bytes()
+        lib().atlas_stream_sync()
+        res["got"] = dy.get().astype(np.float64)
+
+    res = _thread(run)
+    assert res["code"] == 0 and res["error"] == 0 and res["bytes"] == 0
+    w64 = (data.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    x64 = x.astype(np.float64)
+    assert np.all(np.abs(res["got"] - x64 @ w64.T) <= _sum_tol(x64, w64))
+
+
+# Streams whose owner has destroyed them by the thread's next call, on another one; four of them have scratch.
+def test_scratch_after_its_stream_is_gone():
+    M, K, n = 4096, 11008, 127
+    print(f"scratch after its stream is gone M={M} K={K} n={n}", flush=True)
+    hip = _hip_runtime()
+    data, _ = _rand_weights("bf16", M, K, 23)
+    x = np.random.default_rng(24).standard_normal((n, K), np.float32)
+
+    def run(res):
+        streams = [C.c_void_p() for _ in range(6)]
+        dw, dx = Dev(data), Dev(x)
+        for st in streams:
+            assert hip.hipStreamCreate(C.byref(st)) == 0
+        res["got"], res["bytes"] = [], []
+        for st in streams:
+            dy = Dev(np.full((n, M), np.nan, np.float32))
+            lib().atlas_set_thread_stream(st)
+            assert lib().atlas_gemm_skinny_f32(1, dw.ptr, None, 0, dx.ptr, dy.ptr, M, n, K) == 0
+            lib().atlas_stream_sync()
+            res["got"].append(dy.get())
+            res["bytes"].append(lib().atlas_thread_scratch_bytes())
+            lib().atlas_clear_thread_stream()
+            assert hip.hipStreamDestroy(st) == 0
+
+    res = _thread(run)
+    assert all(np.array_equal(g, res["got"][0]) for g in res["got"])
+    assert res["bytes"] == [min(i, 4) * res["bytes"][0] for i in range(1, 7)]
