@@ -850,8 +850,11 @@ int gemm_rows_launch(const GemvArgs& a, hipStream_t st) {
     PgPlan p = pg_plan(a.fmt, a.M, a.N, a.K);
     float* partial = nullptr;
     const size_t split = (size_t)a.N * a.M * sizeof(float);
-    const size_t need = p.splits > 1 ? p.splits * split : 0, hold = a.partial ? need : scratch_to_hold(a);
-    if (std::max(need, hold) > 0 && skinny_partial_for(a, std::max(need, hold), &partial)) {
+    const size_t need = p.splits > 1 ? p.splits * split : 0;
+    const size_t hold = a.partial ? need : std::max(need, scratch_to_hold(a));
+    // (an unsplit call touches the scratch only to make it large enough)
+    const bool ask = need > 0 || (hold > 0 && hold > thread_scratch_held(SCR_GEMM));
+    if (ask && skinny_partial_for(a, hold, &partial)) {
         // Not to be had (no memory, or a capture on a thread that made no such
         // call before it): what there is takes fewer splits, or none.
         clear_error();
