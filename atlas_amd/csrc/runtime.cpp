@@ -31,7 +31,7 @@ constexpr int kScratchDevices = 16;
 // on two streams do not meet in it; beyond this many the one used longest ago
 // changes hands after a device synchronisation.  (The other streams' handles are
 // only compared: their owners may have destroyed them, and HIP crashes on one.)
-constexpr int kScratchStreams = 4;
+constexpr int kScratchStreams = 8;
 struct ScratchBuf {
     void* p = nullptr;
     size_t cap = 0;

@@ -40,7 +40,7 @@
  * of a 7B matrix.)  A graph's launches use the scratch that
  * its calls were captured with, which stays until the thread exits: order
  * them with that thread's other calls.  A thread that calls on several
- * streams has scratch for each of up to four; a fifth takes over the one used
+ * streams has scratch for each of up to eight; a ninth takes over the one used
  * longest ago after a device synchronisation.
  */
 #ifndef ATLAS_KERNELS_H
